@@ -227,12 +227,13 @@ sre_status sre_adjoint(sre_engine *e, const double *dLdE, const double *d_dLdF,
 
 typedef struct {
   int force_lanes;      /* lanes per atom in the force kernel: 1,2,4,8,16 */
-  int build_lanes;      /* lanes per atom in the list build */
+  int build_lanes;      /* 1,2,4,8,16; kept for callers that set it: the list build
+                           takes a few atoms per wavefront at any value */
   int block;            /* threads per block of the force kernel: 64..1024 */
   float cell_xy;        /* cell edge in x,y as a multiple of (rc_min + skin) */
   float cell_z;         /* cell edge in z as a multiple of (rc_min + skin) */
-  int build_mode;       /* 0: per-atom column search (build_lanes lanes per atom);
-                           1: one wavefront per 64-atom tile of a cell column */
+  int build_mode;       /* 0: column search, 4 or 8 atoms per wavefront on the matrix
+                           cores; 1: one wavefront per 64-atom tile of a cell column */
   int xcd_remap;        /* 1: map contiguous atom ranges to each XCD (L2 locality) */
   int force_unroll;     /* list rows per group in the mixed force kernel: 1, 2, 4;
                            FP64 form: 1 = the mixed kernel's pipelined loop,

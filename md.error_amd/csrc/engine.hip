@@ -116,6 +116,7 @@ struct sre_engine {
   int *d_start = nullptr;
   int start_cap = 0;
   int n_cols = 0;                  // (x, y) cell columns over all replicas
+  bool build_images = false;       // list build over second images (build_needs_images)
   uint32_t *d_tiles_per_col = nullptr, *d_tile_off = nullptr, *d_tile_tmp = nullptr;
   int tile_cap = 0;
   uint4 *d_pos4 = nullptr, *d_backup = nullptr;  // backup: caller order
@@ -751,6 +752,7 @@ static sre_status prepare_tables(sre_engine *e) {
   }
   // cell grids
   long long cells = 0, cols = 0;
+  e->build_images = false;
   for (int r = 0; r < e->n_rep; ++r) {
     RepInfo &R = e->reps[r];
     const float rlmax = R.rc_max + e->skin;
@@ -760,6 +762,7 @@ static sre_status prepare_tables(sre_engine *e) {
                     "replica %d: rc_max + skin = %g is not below half the box "
                     "edge %d (%g)", r, rlmax, d, R.L[d]);
     choose_cell_grid(R, e->skin, e->tune.cell_xy, e->tune.cell_z);
+    e->build_images |= build_needs_images(R, e->skin);
     R.cell_off = (int)cells;
     R.col_off = (int)cols;
     cells += (long long)R.nc[0] * R.nc[1] * R.nc[2];
@@ -912,7 +915,7 @@ static std::vector<unsigned char> rebuild_signature(const sre_engine *e,
                       e->tune.force_mode,
                       e->tune.force_lanes, e->n_types, e->pos_stride, n_parts,
                       (e->tail_bins > 0 && e->tail_mode == SRE_TAIL_EXACT) ? 1 : 0,
-                      e->rc_explicit ? 1 : 0};
+                      e->rc_explicit ? 1 : 0, e->build_images ? 1 : 0};
   put(ints, sizeof ints);
   put(&e->skin, sizeof e->skin);
   const void *ptrs[] = {e->d_pos, e->d_rep_of, e->d_reps, e->sb.key_a, e->sb.key_b,
@@ -945,9 +948,9 @@ static void enqueue_build(sre_engine *e, hipStream_t st) {
                        e->d_list, e->d_nnb, e->d_build_part, e->d_tiles_per_col,
                        e->d_tile_off, e->d_tile_tmp, st);
   else
-    launch_build_list(e->tune.build_lanes, e->tune.force_lanes, N, e->d_pos4,
+    launch_build_list(e->tune.force_lanes, e->build_images, N, e->d_pos4,
                       e->d_rcut, e->d_reps, e->d_start, e->skin, e->cap,
-                      e->d_list, e->d_nnb, e->d_build_part, st);
+                      e->d_list, e->list_size, e->d_nnb, e->d_build_part, st);
 }
 
 // The device part of a rebuild (capturable, no host decisions): cell keys,
@@ -1027,8 +1030,7 @@ static sre_status do_rebuild(sre_engine *e) {
     }
     cap = round_up((int)guess, e->tune.force_lanes);
   }
-  const int n_parts = build_part_count(e->tune.build_mode, N, e->tune.build_lanes,
-                                       e->n_cols);
+  const int n_parts = build_part_count(e->tune.build_mode, N, e->n_cols);
   if (e->build_part_cap < n_parts) {
     dfree(e->d_build_part);
     HIP_TRY(dalloc(&e->d_build_part, n_parts));
@@ -1148,11 +1150,9 @@ static ForceArgs force_args(sre_engine *e, bool atom_stats) {
   a.err_flag = e->d_flags + 1;
   a.ctr_in = nullptr;
   a.ctr_out = nullptr;
-  // the per-atom builder writes one (longest list, total) pair per wave of
-  // build_lanes lanes per atom: the force kernel's waves when the lane
-  // counts agree
-  a.wave_len = (e->tune.build_mode == 0 && e->tune.build_lanes == e->list_lanes)
-                   ? e->d_build_part : nullptr;
+  // the list build writes one (longest list, total) pair per 16 atoms: the
+  // force kernel's waves with 4 lanes per atom
+  a.wave_len = (e->tune.build_mode == 0 && e->list_lanes == 4) ? e->d_build_part : nullptr;
   a.xcd_remap = e->tune.xcd_remap;
   a.has_shift = e->has_shift ? 1 : 0;
   // persistent launch: whole blocks of the tuned size
@@ -1492,8 +1492,7 @@ extern "C" sre_status sre_adjoint(sre_engine *e, const double *dLdE,
   a.cap = e->cap;
   a.n_rep = e->n_rep;
   a.list_len = e->list_size;
-  a.wave_len = (e->tune.build_mode == 0 && e->tune.build_lanes == e->list_lanes)
-                   ? e->d_build_part : nullptr;
+  a.wave_len = (e->tune.build_mode == 0 && e->list_lanes == 4) ? e->d_build_part : nullptr;
   a.pos4 = e->d_pos4;
   a.rcut = e->d_rcut;
   a.nnb = e->d_nnb;
@@ -1696,18 +1695,16 @@ extern "C" sre_status sre_autotune(sre_engine *e, unsigned flags,
   // phase 1: binning + list build
   const float cells_xy[] = {0.35f, 0.5f, 0.7f, 1.0f};
   const float cells_z[] = {0.2f, 0.25f, 0.35f, 0.5f};
-  // (build_mode, build_lanes): per-atom search with 4/8/16 lanes, or tiles
-  const int builds[][2] = {{0, 4}, {0, 8}, {0, 16}, {1, 8}};
+  const int builds[] = {0, 1};
   sre_tuning best = e->tune;
   double best_ms = 1e30;
   for (float cxy : cells_xy)
     for (float cz : cells_z)
-      for (const auto &bd : builds) {
+      for (int bd : builds) {
         sre_tuning t = e->tune;
         t.cell_xy = cxy;
         t.cell_z = cz;
-        t.build_mode = bd[0];
-        t.build_lanes = bd[1];
+        t.build_mode = bd;
         sre_status s = sre_set_tuning(e, &t);
         if (s != SRE_OK) return s;
         s = do_rebuild(e);
@@ -2156,8 +2153,7 @@ extern "C" sre_status sre_run_segments(sre_engine *e, unsigned flags, int n_segm
   HIP_TRY(hipSetDevice(e->device));
   // the captured rebuild must match the current layout; otherwise one
   // ordinary rebuild captures it again
-  const int n_parts = build_part_count(e->tune.build_mode, e->n_atoms,
-                                       e->tune.build_lanes, e->n_cols);
+  const int n_parts = build_part_count(e->tune.build_mode, e->n_atoms, e->n_cols);
   if (!e->rebuild_exec || rebuild_signature(e, n_parts) != e->rebuild_sig) {
     sre_status s = do_rebuild(e);
     if (s != SRE_OK) return s;

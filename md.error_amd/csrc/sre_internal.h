@@ -44,6 +44,7 @@ struct RepInfo {
   double qd[3];     // L * 2^-32 in FP64
   int nc[3];        // cell grid
   float h[3];       // cell edges L / nc
+  uint32_t half_cell[2];   // half a cell edge along x, y in lattice units (2^31 / nc, floor)
   int cell_off;     // first global cell id of this replica
   int col_off;      // first global cell column (x, y) of this replica
   int atom_off;     // first atom (caller order and sorted order)
@@ -79,6 +80,7 @@ inline void choose_cell_grid(RepInfo &R, float skin, float cell_xy, float cell_z
   for (int d = 0; d < 3; ++d) {
     R.nc[d] = nc[d];
     R.h[d] = R.L[d] / (float)nc[d];
+    if (d < 2) R.half_cell[d] = 0x80000000u / (uint32_t)nc[d];
   }
 }
 
@@ -368,14 +370,17 @@ void launch_assign_rc(int n, const float *pos, int stride, const int *rep_of,
                       const RepInfo *reps, const float *rc_table,
                       const uint32_t *inv_perm, float *rc_atom, float *rcut,
                       hipStream_t st);
-// Both builders write one (longest list, total length) pair per wavefront to
-// part[] (build_part_count entries, every one written by every launch);
-// launch_rebuild_info reduces them.
-int build_part_count(int mode, int n, int lanes, int n_cols);
-void launch_build_list(int lanes, int force_lanes, int n, const uint4 *pos4,
+// Both builders write (longest list, total length) pairs to part[]
+// (build_part_count entries, every one written by every launch; mode 0: one
+// pair per 16 sorted atoms); launch_rebuild_info reduces them.
+int build_part_count(int mode, int n, int n_cols);
+// images: some replica's cells are so large a part of its box that a tile's
+// atoms may see a candidate's second image along x or y (build_needs_images)
+bool build_needs_images(const RepInfo &R, float skin);
+void launch_build_list(int force_lanes, bool images, int n, const uint4 *pos4,
                        const float *rcut, const RepInfo *reps, const int *start,
-                       float skin, int cap, int *list, int *nnb, int2 *part,
-                       hipStream_t st);
+                       float skin, int cap, int *list, size_t list_len, int *nnb,
+                       int2 *part, hipStream_t st);
 // Tiles of <= tile atoms inside one cell column: tiles_per_col and tile_off
 // (n_cols each) filled on the device from the cell offsets.
 void launch_tile_map(int n_cols, int n_rep, const RepInfo *reps, const int *start,
@@ -552,8 +557,8 @@ struct ForceArgs {
   // step from *ctr_in); NULL = none
   const uint64_t *ctr_in;
   uint64_t *ctr_out;
-  const int2 *wave_len;        // per force wavefront: (longest list, total) from a
-                               // list build of the same tiling, or NULL
+  const int2 *wave_len;        // per force wavefront: (longest list, total) from the
+                               // list build when its tiles have 16 atoms, or NULL
   int xcd_remap;               // 1: contiguous block ranges per XCD
   int has_shift;               // some pair type has a nonzero energy shift
   int persist_waves;           // mixed form: > 0 = persistent launch of that many

@@ -147,7 +147,7 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   const int A = kWave / T;
   const size_t waves = (size_t)(N + A - 1) / A;
   const size_t list_len = waves * (size_t)cap * A + (size_t)kListPadRows * kWave;
-  const int n_parts = build_part_count(0, N, T, 0);
+  const int n_parts = build_part_count(0, N, 0);
   const size_t cc = radix_counts_capacity(N, key_bits);
 
   Carve c{base};
@@ -209,7 +209,7 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   launch_gather_sorted(N, (int)cells, sb.key_a, sb.val_a, d_xyz, stride, types, d_rep_of,
                        d_reps, d_rc, n_types, d_start, d_pos4, d_backup, d_inv_perm,
                        nullptr, d_rcut, d_tail_idx, nullptr, st);
-  launch_build_list(T, T, N, d_pos4, d_rcut, d_reps, d_start, skin, cap, d_list, d_nnb,
+  launch_build_list(T, build_needs_images(R, skin), N, d_pos4, d_rcut, d_reps, d_start, skin, cap, d_list, list_len, d_nnb,
                     d_build_part, st);
   launch_rebuild_info(n_parts, d_build_part, d_counters, 0, nullptr, 0, nullptr, st);
   HIP_TRY(hipGetLastError());
