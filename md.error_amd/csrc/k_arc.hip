@@ -15,8 +15,12 @@
 //    Gauss-Legendre, panel width <= 1/8 and <= 1/(8k)), recording the running
 //    integral at every candidate, so all candidates cost one pass;
 //  * transforms: the grid edges are odd (the reference makes them so), so a
-//    3-D DFT is three passes of direct per-axis DFTs (one thread per output
-//    element, twiddles from an exact table), O(nele * (nx + ny + nz));
+//    3-D DFT is three passes of direct per-axis DFTs, O(nele * (nx + ny + nz)).
+//    With P_j = x_j + x_{n-j}, M_j = x_j - x_{n-j} the outputs k and n - k
+//    share two real sums over half the line, C_k = sum P_j cos and S_k = sum
+//    M_j sin: real matrix products of a twiddle table with many lines, done on
+//    the FP64 matrix cores (k_arc_axis), a quarter of the direct operations.
+//    Edges above kArcAxisMax take one thread per output (k_arc_dft);
 //  * the four inverse transforms per candidate are packed into two complex
 //    ones (every output is real: Z1 = (S1 - kx G) rho_k -> e1 + i e2x,
 //    Z2 = (i ky - kz) G rho_k -> e2y + i e2z), all candidates in one batch.
@@ -390,6 +394,220 @@ __global__ void k_arc_density(int nele, double norm, const unsigned *counts,
   if (i < nele) rho[i] = (double)counts[i] / norm;
 }
 
+// ---- one axis of the transforms on the matrix cores ----------------------
+//
+// A block takes 8 NT neighbouring lines of one axis, for one transform or for
+// the pair (2c, 2c + 1) of candidate c (two groups of wavefronts, one each):
+// the lines go to LDS, are combined in place to P_j and M_j, and wavefront kt
+// of a group forms the outputs k in [16 kt, 16 kt + 16) and their mirrors:
+// D[16 k x 16 columns] += T[16 k x 4 j] X[4 j x 16 columns] with
+// v_mfma_f64_16x16x4, a column being the real or the imaginary part of a line.
+// IN: what a line element is before the first pass (the packing of the error
+// or pressure kernels with rho_k, or a real grid); OUT: what becomes of it
+// after the last one (the error estimate of the candidate).  In place: a
+// block reads its lines whole before it writes them.
+// What bounds it: memory and cache traffic (per pass of 22 grids of 100 000
+// cells 35 MB in and out); the products are ~0.4e9 FMA per estimate, 10 us at
+// the FP64 rate.  Measured per pass for 11 candidates on 29 x 29 x 119 cells:
+// 21 (packing), 23 and 25 us (error estimate written), 2.3 to 3 TB/s; with one
+// thread per output, 86 us on average and 45 us more for packing, copying and
+// combining in launches of their own.  16 lines per block up to edges of 60
+// (one or two tiles of outputs: enough wavefronts), 8 beyond (the pair of
+// groups stays within 64 KB of LDS up to kArcAxisMax).
+constexpr int kArcAxisMax = 227;    // edge: a pair of groups of 8 lines in 64 KB of LDS
+enum { kArcPlain = 0, kArcReal = 1, kArcErr = 2, kArcPress = 3 };
+struct ArcAxisArgs {
+  ArcGrid g;
+  int axis;
+  int kt, jt;                 // tiles of 16 outputs, of 4 inputs
+  const double *ct, *st;      // cos and sin tables, one wavefront load per tile
+  const double *kx, *ky, *kz; // signed frequency / L per index
+  double sgn;                 // sign of the transform's exponent
+  double scale;               // of rho_k (kArcErr, kArcPress)
+  double inv_vol;             // kArcErr after the last pass
+  double2 *z;                 // the grids
+  const double *rho;          // kArcReal
+  const double *T1, *T2;      // S1, G or I1, I5
+  const double2 *rhok;
+  double *err, *parts;
+};
+
+// tables of axis length n: entry (kt, jt, lane) for k = 16 kt + lane % 16 and
+// j = 1 + 4 jt + lane / 16, zero beyond the half line
+__global__ void k_arc_tables(int n, int kt, int jt, double *ct, double *st) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= kt * jt * kWave) return;
+  const int lane = e % kWave, t = e / kWave;
+  const int k = (t / jt) * 16 + lane % 16, j = 1 + (t % jt) * 4 + lane / 16;
+  const int h = (n - 1) / 2;
+  double s = 0.0, c = 0.0;
+  if (k <= h && j <= h) sincospi(2.0 * (double)((k * j) % n) / (double)n, &s, &c);
+  ct[e] = c;
+  st[e] = s;
+}
+
+__global__ void k_arc_kvec(ArcGrid g, int axis, double *kv) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= g.n[axis]) return;
+  const int f = i <= (g.n[axis] - 1) / 2 ? i : i - g.n[axis];
+  kv[i] = (double)f / g.L[axis];
+}
+
+typedef double sre_f64x4 __attribute__((ext_vector_type(4)));
+
+// the neighbouring lane's value (lane ^ 1)
+__device__ __forceinline__ double lane_x1(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0xB1, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0xB1, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int NT, int IN, int OUT>
+__global__ __launch_bounds__(1024) void k_arc_axis(ArcAxisArgs a) {
+  constexpr int NC = 8 * NT;     // lines per block
+  constexpr int RS = NC + 1;     // LDS row (one j of every line), padded
+  extern __shared__ double2 lds[];
+  const int n = a.g.n[a.axis], h = (n - 1) / 2;
+  const int lines = a.g.nele / n;
+  const int groups = (int)blockDim.x / (kWave * a.kt);
+  const int stride = a.axis == 0 ? a.g.n[1] * a.g.n[2] : (a.axis == 1 ? a.g.n[2] : 1);
+  const int q0 = blockIdx.x * NC;
+  const int b0 = (int)blockIdx.y * groups;     // the first group's transform
+  // a thread copies positions jc, jc + jstep, ... of line c: neighbouring
+  // threads take neighbouring cells (lines of axes 0 and 1, positions of
+  // axis 2); a line past the last one repeats the last
+  const int per = (int)blockDim.x / NC;
+  const int c = a.axis == 2 ? (int)threadIdx.x / per : (int)threadIdx.x % NC;
+  const int jc = a.axis == 2 ? (int)threadIdx.x - c * per : (int)threadIdx.x / NC;
+  const int q = min(q0 + c, lines - 1);
+  const int base = a.axis == 1 ? (q / a.g.n[2]) * a.g.n[1] * a.g.n[2] + q % a.g.n[2]
+                               : (a.axis == 0 ? q : q * n);
+  const size_t grid0 = (size_t)b0 * a.g.nele;
+  // (the packing passes run along axis 0: line q is (iy, iz))
+  const double ky = IN >= kArcErr ? a.ky[q / a.g.n[2]] : 0.0;
+  const double kz = IN >= kArcErr ? a.kz[q % a.g.n[2]] : 0.0;
+  // the element's value in each group's transform
+  auto load = [&](int j, double2 v[2]) {
+    const int cell = base + j * stride;
+    if (IN == kArcReal) {
+      v[0] = make_double2(a.rho[cell], 0.0);
+    } else if (IN == kArcPlain) {
+      v[0] = a.z[grid0 + cell];
+      if (groups == 2) v[1] = a.z[grid0 + a.g.nele + cell];
+    } else {
+      // both transforms of candidate blockIdx.y: Z1 = (S1 - kx G) rho_k and
+      // Z2 = (i ky - kz) G rho_k, or (Kxx + i Kyy) rho_k and Kzz rho_k
+      const double kv[3] = {a.kx[j], ky, kz};
+      const size_t gi = (size_t)blockIdx.y * a.g.nele + cell;
+      const double2 rk = a.rhok[cell];
+      const double2 r = make_double2(rk.x * a.scale, rk.y * a.scale);
+      if (IN == kArcErr) {
+        const double gg = a.T2[gi];
+        const double p = a.T1[gi] - kv[0] * gg;
+        const double br = -kv[2] * gg, bi = kv[1] * gg;
+        v[0] = make_double2(p * r.x, p * r.y);
+        v[1] = make_double2(br * r.x - bi * r.y, br * r.y + bi * r.x);
+      } else {
+        double K[3];
+        pressure_kernel(kv, a.T1[gi], a.T2[gi], K);
+        v[0] = make_double2(K[0] * r.x - K[1] * r.y, K[0] * r.y + K[1] * r.x);
+        v[1] = make_double2(K[2] * r.x, K[2] * r.y);
+      }
+    }
+  };
+  // kU elements per thread in flight: four shorten the packing passes (a real
+  // grid 9.0 -> 6.8 us, one wavefront per block), more than one slows the plain
+  // ones (22 grids of 100 000 cells: 22.9 us with one, 31 with two, 35 with four)
+  constexpr int kU = IN == kArcPlain ? 1 : 4;
+  for (int j0 = jc; j0 < n; j0 += kU * per) {
+    double2 v[kU][2];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (j0 + u * per < n) load(j0 + u * per, v[u]);
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (j0 + u * per < n) {
+        double2 *const dst = lds + (j0 + u * per) * RS + c;
+        dst[0] = v[u][0];
+        if (groups == 2) dst[n * RS] = v[u][1];
+      }
+  }
+  __syncthreads();
+  for (int gr = 0; gr < groups; ++gr)
+    for (int j = 1 + (int)threadIdx.x / NC; j <= h; j += per) {
+      double2 *const line = lds + gr * n * RS + (int)threadIdx.x % NC;
+      double2 *const p = line + j * RS, *const m = line + (n - j) * RS;
+      const double2 x = *p, y = *m;
+      *p = make_double2(x.x + y.x, x.y + y.y);
+      *m = make_double2(x.x - y.x, x.y - y.y);
+    }
+  __syncthreads();
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int gr = wave / a.kt, kt = wave - gr * a.kt;
+  double *const rows = reinterpret_cast<double *>(lds + gr * n * RS);
+  sre_f64x4 C[NT] = {}, S[NT] = {};
+  {
+    const double *ct = a.ct + (size_t)kt * a.jt * kWave + lane;
+    const double *st = a.st + (size_t)kt * a.jt * kWave + lane;
+    for (int jt = 0; jt < a.jt; ++jt) {
+      // (past the half line the table is zero: any row will do)
+      const int j = min(1 + 4 * jt + lane / 16, h);
+      const double *p = rows + (size_t)j * 2 * RS + lane % 16;
+      const double *m = rows + (size_t)(n - j) * 2 * RS + lane % 16;
+      const double cs = ct[jt * kWave], sn = st[jt * kWave];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        C[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cs, p[16 * t], C[t], 0, 0, 0);
+        S[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(sn, m[16 * t], S[t], 0, 0, 0);
+      }
+    }
+  }
+  double x0[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) x0[t] = rows[16 * t + lane % 16];
+  __syncthreads();   // every line has been read
+  // X_k = x_0 + C_k + i sgn S_k and X_{n-k} = x_0 + C_k - i sgn S_k
+  const double sp = (lane & 1) ? a.sgn : -a.sgn;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = kt * 16 + 4 * r + lane / 16;
+      const double u = sp * lane_x1(S[t][r]);
+      const double v = x0[t] + C[t][r];
+      if (k <= h) {
+        rows[(size_t)k * 2 * RS + 16 * t + lane % 16] = v + u;
+        if (k > 0) rows[(size_t)(n - k) * 2 * RS + 16 * t + lane % 16] = v - u;
+      }
+    }
+  __syncthreads();
+  if (q0 + c >= lines) return;
+  for (int j = jc; j < n; j += per) {
+    const int cell = base + j * stride;
+    const double2 *src = lds + j * RS + c;
+    if (OUT == kArcErr) {
+      // error = sqrt(e1 + e2x^2 + e2y^2 + e2z^2), every part divided by V
+      const double2 z1 = src[0], z2 = src[n * RS];
+      const double e1 = z1.x * a.inv_vol, ex = z1.y * a.inv_vol;
+      const double ey = z2.x * a.inv_vol, ez = z2.y * a.inv_vol;
+      const size_t gi = (size_t)blockIdx.y * a.g.nele + cell;
+      a.err[gi] = sqrt(e1 + ex * ex + ey * ey + ez * ez);
+      if (a.parts) {
+        double *p = a.parts + gi * 4;
+        p[0] = e1;
+        p[1] = ex;
+        p[2] = ey;
+        p[3] = ez;
+      }
+    } else {
+      a.z[grid0 + cell] = src[0];
+      if (groups == 2) a.z[grid0 + a.g.nele + cell] = src[n * RS];
+    }
+  }
+}
+
 static unsigned arc_blocks(size_t n) {
   return (unsigned)((n + kArcBlock - 1) / kArcBlock);
 }
@@ -446,6 +664,9 @@ struct sre_arc {
   double *d_I1 = nullptr, *d_I5 = nullptr;  // pressure-kernel integrals [nrc][nele]
   double *d_psum = nullptr;                 // pressure partial sums, 3 per block
   double2 *d_tw[3][2] = {};                 // per axis: forward, backward
+  bool matrix = false;                      // every edge fits k_arc_axis
+  double *d_ct[3] = {}, *d_st[3] = {};      // its tables per axis
+  double *d_kv[3] = {};                     // signed frequency / L per index
   unsigned *d_counts = nullptr;
   int ndata = 0;
   double *d_rho = nullptr;
@@ -465,12 +686,52 @@ struct sre_arc {
 sre_arc::~sre_arc() {
   dfree(d_rcs); dfree(d_S1); dfree(d_G); dfree(d_I1); dfree(d_I5); dfree(d_psum);
   for (auto &a : d_tw) { dfree(a[0]); dfree(a[1]); }
+  for (int d = 0; d < 3; ++d) { dfree(d_ct[d]); dfree(d_st[d]); dfree(d_kv[d]); }
   dfree(d_counts); dfree(d_rho); dfree(d_rhok); dfree(d_zr); dfree(d_za);
   dfree(d_zb); dfree(d_err); dfree(d_parts); dfree(d_idx); dfree(d_idx2);
   dfree(d_rc); dfree(d_res_err); dfree(d_fgrid);
   if (engine_done) (void)hipEventDestroy(engine_done);
   if (deposit_done) (void)hipEventDestroy(deposit_done);
   if (own_stream && stream) (void)hipStreamDestroy(stream);
+}
+
+static int arc_kt(int n) { return ((n - 1) / 2 + 1 + 15) / 16; }
+static int arc_jt(int n) { return ((n - 1) / 2 + 3) / 4; }
+
+// one axis of the forward transform of one grid (pairs = 0) or of `pairs`
+// pairs of grids
+template <int IN, int OUT>
+static void arc_axis(sre_arc *a, ArcAxisArgs args, int axis, int pairs) {
+  const int n = a->g.n[axis], groups = pairs > 0 ? 2 : 1;
+  args.g = a->g;
+  args.axis = axis;
+  args.kt = arc_kt(n);
+  args.jt = arc_jt(n);
+  args.ct = a->d_ct[axis];
+  args.st = a->d_st[axis];
+  args.kx = a->d_kv[0];
+  args.ky = a->d_kv[1];
+  args.kz = a->d_kv[2];
+  const int lines = a->g.nele / n;
+  const dim3 b(kWave * args.kt * groups);
+  const int ny = pairs > 0 ? pairs : 1;
+  if (n <= 60)
+    hipLaunchKernelGGL((k_arc_axis<2, IN, OUT>), dim3((lines + 15) / 16, ny), b,
+                       (size_t)groups * n * 17 * sizeof(double2), a->stream, args);
+  else
+    hipLaunchKernelGGL((k_arc_axis<1, IN, OUT>), dim3((lines + 7) / 8, ny), b,
+                       (size_t)groups * n * 9 * sizeof(double2), a->stream, args);
+}
+
+// rho_k of the current density
+static void arc_forward(sre_arc *a) {
+  ArcAxisArgs f{};
+  f.sgn = -1.0;
+  f.z = a->d_rhok;
+  f.rho = a->d_rho;
+  arc_axis<kArcReal, kArcPlain>(a, f, 0, 0);
+  arc_axis<kArcPlain, kArcPlain>(a, f, 1, 0);
+  arc_axis<kArcPlain, kArcPlain>(a, f, 2, 0);
 }
 
 // batched 3-D DFT of za (batch grids) in place (zb scratch of the same size)
@@ -545,6 +806,20 @@ extern "C" sre_status sre_arc_create(sre_arc **out, const double box[3],
         hipLaunchKernelGGL(k_arc_twiddle, dim3(arc_blocks(a->g.n[d])), dim3(kArcBlock),
                            0, a->stream, a->g.n[d], dir == 0 ? -1 : 1, a->d_tw[d][dir]);
       }
+    a->matrix = true;
+    for (int d = 0; d < 3; ++d) a->matrix &= a->g.n[d] <= kArcAxisMax;
+    for (int d = 0; a->matrix && d < 3; ++d) {
+      const int n = a->g.n[d], kt = arc_kt(n), jt = arc_jt(n);
+      const size_t m = (size_t)kt * jt * kWave;
+      HIP_TRY(dalloc(&a->d_ct[d], m + 1));     // (an edge of one cell has no entries)
+      HIP_TRY(dalloc(&a->d_st[d], m + 1));
+      HIP_TRY(dalloc(&a->d_kv[d], n));
+      if (m > 0)
+        hipLaunchKernelGGL(k_arc_tables, dim3(arc_blocks(m)), dim3(kArcBlock), 0, a->stream,
+                           n, kt, jt, a->d_ct[d], a->d_st[d]);
+      hipLaunchKernelGGL(k_arc_kvec, dim3(arc_blocks(n)), dim3(kArcBlock), 0, a->stream,
+                         a->g, d, a->d_kv[d]);
+    }
     HIP_TRY(hipMemsetAsync(a->d_counts, 0, sizeof(unsigned) * nele, a->stream));
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(a->stream));
@@ -584,7 +859,7 @@ extern "C" sre_status sre_arc_set_candidates(sre_arc *a, double rcmin, double rc
   HIP_TRY(dalloc(&a->d_I1, tab));
   HIP_TRY(dalloc(&a->d_I5, tab));
   HIP_TRY(dalloc(&a->d_za, 2 * tab));
-  HIP_TRY(dalloc(&a->d_zb, 2 * tab));
+  if (!a->matrix) HIP_TRY(dalloc(&a->d_zb, 2 * tab));
   HIP_TRY(dalloc(&a->d_err, tab));
   HIP_TRY(hipMemcpyAsync(a->d_rcs, rcs.data(), sizeof(double) * nrc,
                          hipMemcpyHostToDevice, a->stream));
@@ -709,7 +984,29 @@ extern "C" sre_status sre_arc_cal_error(sre_arc *a, int keep_parts) {
   const int nrc = (int)a->rcs.size();
   const size_t tab = (size_t)nrc * g.nele;
   const double vol = g.L[0] * g.L[1] * g.L[2];
+  if (keep_parts && !a->d_parts) HIP_TRY(dalloc(&a->d_parts, 4 * tab));
   // rho_k = FFT(rho) (forward: exp(-2 pi i ...)), scaled by V / nele in pack
+  if (a->matrix) {
+    arc_forward(a);
+    ArcAxisArgs e{};
+    e.sgn = 1.0;
+    e.scale = vol / g.nele;
+    e.inv_vol = 1.0 / vol;
+    e.z = a->d_za;
+    e.T1 = a->d_S1;
+    e.T2 = a->d_G;
+    e.rhok = a->d_rhok;
+    e.err = a->d_err;
+    e.parts = keep_parts ? a->d_parts : nullptr;
+    arc_axis<kArcErr, kArcPlain>(a, e, 0, nrc);
+    arc_axis<kArcPlain, kArcPlain>(a, e, 1, nrc);
+    arc_axis<kArcPlain, kArcErr>(a, e, 2, nrc);
+    HIP_TRY(hipGetLastError());
+    a->err_valid = true;
+    a->parts_valid = keep_parts != 0;
+    a->rc_valid = false;
+    return SRE_OK;
+  }
   hipLaunchKernelGGL(k_arc_real_to_complex, dim3(arc_blocks(g.nele)), dim3(kArcBlock),
                      0, a->stream, g.nele, a->d_rho, a->d_rhok);
   s = arc_dft3(a, 1, 0, a->d_rhok, a->d_zr);
@@ -718,7 +1015,6 @@ extern "C" sre_status sre_arc_cal_error(sre_arc *a, int keep_parts) {
                      g, nrc, vol / g.nele, a->d_S1, a->d_G, a->d_rhok, a->d_za);
   s = arc_dft3(a, 2 * nrc, 1, a->d_za, a->d_zb);
   if (s != SRE_OK) return s;
-  if (keep_parts && !a->d_parts) HIP_TRY(dalloc(&a->d_parts, 4 * tab));
   hipLaunchKernelGGL(k_arc_combine, dim3(arc_blocks(tab)), dim3(kArcBlock), 0,
                      a->stream, g, nrc, 1.0 / vol, a->d_za, a->d_err,
                      keep_parts ? a->d_parts : nullptr);
@@ -837,15 +1133,29 @@ extern "C" sre_status sre_arc_pressure(sre_arc *a, double *p) {
   const int nrc = (int)a->rcs.size();
   const size_t tab = (size_t)nrc * g.nele;
   const double vol = g.L[0] * g.L[1] * g.L[2];
-  hipLaunchKernelGGL(k_arc_real_to_complex, dim3(arc_blocks(g.nele)), dim3(kArcBlock),
-                     0, a->stream, g.nele, a->d_rho, a->d_rhok);
-  s = arc_dft3(a, 1, 0, a->d_rhok, a->d_zr);
-  if (s != SRE_OK) return s;
-  hipLaunchKernelGGL(k_arc_pack_pressure, dim3(arc_blocks(tab)), dim3(kArcBlock), 0,
-                     a->stream, g, nrc, vol / g.nele, a->d_I1, a->d_I5, a->d_rhok,
-                     a->d_za);
-  s = arc_dft3(a, 2 * nrc, 1, a->d_za, a->d_zb);
-  if (s != SRE_OK) return s;
+  if (a->matrix) {
+    arc_forward(a);
+    ArcAxisArgs e{};
+    e.sgn = 1.0;
+    e.scale = vol / g.nele;
+    e.z = a->d_za;
+    e.T1 = a->d_I1;
+    e.T2 = a->d_I5;
+    e.rhok = a->d_rhok;
+    arc_axis<kArcPress, kArcPlain>(a, e, 0, nrc);
+    arc_axis<kArcPlain, kArcPlain>(a, e, 1, nrc);
+    arc_axis<kArcPlain, kArcPlain>(a, e, 2, nrc);
+  } else {
+    hipLaunchKernelGGL(k_arc_real_to_complex, dim3(arc_blocks(g.nele)), dim3(kArcBlock),
+                       0, a->stream, g.nele, a->d_rho, a->d_rhok);
+    s = arc_dft3(a, 1, 0, a->d_rhok, a->d_zr);
+    if (s != SRE_OK) return s;
+    hipLaunchKernelGGL(k_arc_pack_pressure, dim3(arc_blocks(tab)), dim3(kArcBlock), 0,
+                       a->stream, g, nrc, vol / g.nele, a->d_I1, a->d_I5, a->d_rhok,
+                       a->d_za);
+    s = arc_dft3(a, 2 * nrc, 1, a->d_za, a->d_zb);
+    if (s != SRE_OK) return s;
+  }
   const unsigned nb = arc_blocks(g.nele);
   hipLaunchKernelGGL(k_arc_pressure_sum, dim3(nb), dim3(kArcBlock), 0, a->stream, g,
                      a->d_idx, a->d_rho, a->d_za, a->d_psum);
