@@ -151,14 +151,6 @@ def run_form(w, precision, steps, warmup, every, torch, Engine, autotune=False):
     # force kernel alone, back-to-back launches on the same stream (HIP events)
     e.time_compute(20, stats=True, tail=True)      # warm the clocks and caches
     k_ms = e.time_compute(200, stats=True, tail=True)
-    k_piped_ms = None
-    if precision == "fp64":
-        # the FP64 form in the mixed kernel's pipelined structure, same sums
-        plain = e.tuning()
-        e.set_tuning(force_unroll=1)
-        e.time_compute(20, stats=True, tail=True)
-        k_piped_ms = e.time_compute(200, stats=True, tail=True)
-        e.set_tuning(**plain)
     k_cells_ms = None
     if precision == "mixed":
         # the cell-window form without a list (LDS-staged candidates, bitwise
@@ -179,7 +171,7 @@ def run_form(w, precision, steps, warmup, every, torch, Engine, autotune=False):
     return dict(engine=e, pos=pos, wall_s=wall, gpu_ms=gpu_ms, pairs=pairs, warm=warm,
                 rebuilds=rebuilds, force_ms=k_ms, n_list=nl, n_in_rc=nin, max_list=mx,
                 force_us_dist=dist, rebuild_ms=rb_ms, autotune_s=tune_s,
-                force_piped_ms=k_piped_ms, force_cells_ms=k_cells_ms,
+                force_cells_ms=k_cells_ms,
                 pair_evals_per_s=pairs / wall, ms_per_step=1e3 * wall / steps)
 
 
@@ -638,12 +630,10 @@ def main():
             "value": round(fp64["pair_evals_per_s"], 1), "ms_per_step": round(fp64["ms_per_step"], 5),
             "force_kernel_us": round(fp64["force_ms"] * 1e3, 3),
             "force_kernel_us_per_launch": fp64["force_us_dist"],
-            "rebuild_us": round(fp64["rebuild_ms"] * 1e3, 1),
-            "force_kernel_us_pipelined": round(fp64["force_piped_ms"] * 1e3, 3)}
+            "rebuild_us": round(fp64["rebuild_ms"] * 1e3, 1)}
         result["speedup_mixed_vs_fp64"] = {
             "whole_step": round(mixed["pair_evals_per_s"] / fp64["pair_evals_per_s"], 3),
-            "force_kernel": round(fp64["force_ms"] / mixed["force_ms"], 3),
-            "force_kernel_vs_pipelined_fp64": round(fp64["force_piped_ms"] / mixed["force_ms"], 3)}
+            "force_kernel": round(fp64["force_ms"] / mixed["force_ms"], 3)}
     print(json.dumps(result), flush=True)
 
 

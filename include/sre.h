@@ -235,9 +235,8 @@ typedef struct {
   int build_mode;       /* 0: column search, 4 or 8 atoms per wavefront on the matrix
                            cores; 1: one wavefront per 64-atom tile of a cell column */
   int xcd_remap;        /* 1: map contiguous atom ranges to each XCD (L2 locality) */
-  int force_unroll;     /* list rows per group in the mixed force kernel: 1, 2, 4;
-                           FP64 form: 1 = the mixed kernel's pipelined loop,
-                           2 or 4 = the plain per-lane loop (same sums) */
+  int force_unroll;     /* list rows per group in the mixed force kernel: 1, 2, 4
+                           (the FP64 form takes one row per group at any value) */
   int persistent;       /* mixed force kernel: 0 = one wavefront per tile of 64/lanes
                            atoms (flat launch over all replicas); k = 1..16: a
                            persistent launch of k wavefronts per SIMD, each taking a

@@ -843,102 +843,37 @@ void launch_force_cells(bool stats, bool tail, const ForceArgs &a, const CellWin
 
 // --------------------------------------------------------------- FP64 ----
 
-template <int T, bool STATS, bool TAIL, bool MULTI, bool NEXT>
-__global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
-  if (a.ctr_out && blockIdx.x == 0 && threadIdx.x == 0) *a.ctr_out = *a.ctr_in + 1;
-  __shared__ PairParamD sp[MULTI ? kMaxPairTypes : 1];
-  if (MULTI) {
-    for (int t = threadIdx.x; t < a.n_types * a.n_types; t += blockDim.x)
-      sp[t] = a.paramsd[t];
-    __syncthreads();
-  }
-  constexpr int A = kWave / T;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int l = lane % T;
-  int bid, nb;
-  if (!force_block<NEXT>(a, &bid, &nb)) return;
-  const int blk = a.xcd_remap ? xcd_block(bid, nb) : bid;
-  const int wave = (blk * blockDim.x + threadIdx.x) / kWave;
-  const int s = wave * A + lane / T;
-  const bool act = s < a.n;
-  const int s0 = wave * A;
-  if (s0 >= a.n) return;
-  const int sa = act ? s : s0;
-  const uint4 pi = a.pos4[sa];
-  const float4 ri = a.res4[sa];
-  const float rc = a.rcut[sa];
-  const int nn = act ? a.nnb[sa] : 0;
+// 1/x to the last bit or two: two Newton steps on the hardware's estimate (a
+// correctly rounded division takes twice the instructions, for scaling and
+// fix-up that a squared distance inside a cutoff cannot need)
+__device__ __forceinline__ double rcp64(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
 
-  double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
-  if (act) {
-    const RepInfo &R = a.reps[pi.w >> 8];
-    const float qx = R.q[0], qy = R.q[1], qz = R.q[2];
-    const double qdx = R.qd[0], qdy = R.qd[1], qdz = R.qd[2];
-    const float rc2 = rc * rc;
-    const int ti = (int)(pi.w & 0xffu) * a.n_types;
-    const int iters = (nn + T - 1) / T;
-    PairParamD P = a.paramsd[0];
-    const int *lp = a.list + (size_t)wave * (size_t)a.cap * A + lane;
-    for (int m = 0; m < iters; ++m) {
-      const int k = m * T + l;
-      const bool v = k < nn;
-      const int j = v ? lp[(size_t)m * kWave] : s;
-      const uint4 pj = a.pos4[j];
-      // the pair set is decided by the FP32 predicate shared with the mixed path
-      const float d2f = dist2(disp(pj.x, pi.x, qx), disp(pj.y, pi.y, qy),
-                              disp(pj.z, pi.z, qz));
-      const bool in = v && (d2f < rc2);
-      if (MULTI) P = sp[ti + (int)(pj.w & 0xffu)];
-      const float4 rj = a.res4[j];
-      const double dx = (double)(int32_t)(pj.x - pi.x) * qdx + ((double)rj.x - (double)ri.x);
-      const double dy = (double)(int32_t)(pj.y - pi.y) * qdy + ((double)rj.y - (double)ri.y);
-      const double dz = (double)(int32_t)(pj.z - pi.z) * qdz + ((double)rj.z - (double)ri.z);
-      const double d2 = dx * dx + dy * dy + dz * dz;
-      const double ri2 = in ? 1.0 / d2 : 0.0;
-      const double ri6 = ri2 * ri2 * ri2;
-      const double fs = ri2 * ri6 * (P.B6 - P.A12 * ri6);
-      fx += fs * dx;
-      fy += fs * dy;
-      fz += fs * dz;
-      if (STATS) {
-        e += in ? ri6 * (P.A * ri6 - P.B) + P.shift : 0.0;
-        wx += fs * dx * dx;
-        wy += fs * dy * dy;
-        wz += fs * dz * dz;
-      }
-    }
-  }
-  fx = group_sum(fx, T);
-  fy = group_sum(fy, T);
-  fz = group_sum(fz, T);
-  double E = 0.0, Wx = 0.0, Wy = 0.0, Wz = 0.0;
+// One pair of the FP64 form: displacement d (x_j - x_i), inside the cutoff or
+// not, added to the sums
+template <bool STATS>
+__device__ __forceinline__ void pair_fp64(double dx, double dy, double dz, bool in,
+                                          const PairParamD &P, double &fx, double &fy,
+                                          double &fz, double &e, double &wx, double &wy,
+                                          double &wz) {
+  const double d2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+  // coincident atoms: an infinite energy, as of a division (nonzero d2 is
+  // above 1e-90, the squares of the residuals' smallest steps)
+  const double ri2 = in ? rcp64(fmax(d2, 1e-200)) : 0.0;
+  const double ri6 = ri2 * ri2 * ri2;
+  const double fs = ri2 * ri6 * __builtin_fma(-P.A12, ri6, P.B6);
+  fx = __builtin_fma(fs, dx, fx);
+  fy = __builtin_fma(fs, dy, fy);
+  fz = __builtin_fma(fs, dz, fz);
   if (STATS) {
-    E = group_sum(e, T) * 0.5;
-    Wx = group_sum(wx, T) * 0.5;
-    Wy = group_sum(wy, T) * 0.5;
-    Wz = group_sum(wz, T) * 0.5;
-  }
-  const bool own = act && l == 0;
-  if (own) {
-    if (TAIL) {
-      double2 tv = make_double2(0.0, 0.0);
-      if (a.tail_atom) {
-        tv = a.tail_atom[s];
-      } else {
-        const int ti = a.tail_idx[s];
-        if (ti >= 0) tv = a.tail[ti];
-      }
-      fz += tv.x;
-      E += tv.y;
-    }
-    a.fxd[s] = fx;
-    a.fyd[s] = fy;
-    a.fzd[s] = fz;
-    if (STATS) {
-      double2 *d = reinterpret_cast<double2 *>(a.atom_stats + (size_t)s * 4);
-      d[0] = make_double2(E, Wx);
-      d[1] = make_double2(Wy, Wz);
-    }
+    const double t = __builtin_fma(P.A, ri6, -P.B);
+    e += in ? __builtin_fma(ri6, t, P.shift) : 0.0;
+    wx = __builtin_fma(fs * dx, dx, wx);
+    wy = __builtin_fma(fs * dy, dy, wy);
+    wz = __builtin_fma(fs * dz, dz, wz);
   }
 }
 
@@ -946,10 +881,13 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
 // software-pipelined loop (list rows two groups ahead through a per-wave
 // resource, indexed gathers of the next group's lattice positions and
 // sub-lattice residuals, one list row per group), the same pair set (the
-// FP32 predicate) and FP64 arithmetic and sums as k_force_fp64.  Selected
-// for the FP64 form by force_unroll = 1; measured beside the plain form.
+// FP32 predicate), FP64 arithmetic and sums.  What bounds it: FP64 VALU issue
+// and, with few atoms, one wavefront's chain of rows.  A plain loop (direct
+// loads, per-lane trip count, correctly rounded division, separate multiply
+// and add) took 21.9 us on the 64k slab (8 lanes per atom, energy and virial),
+// 7.3 at 4 000 atoms and 280 at 1 million; this one 16.7, 5.1 and 221 us.
 template <int T, bool STATS, bool TAIL, bool MULTI, bool NEXT>
-__global__ __launch_bounds__(256) void k_force_fp64_piped(ForceArgs a) {
+__global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
   if (a.ctr_out && blockIdx.x == 0 && threadIdx.x == 0) *a.ctr_out = *a.ctr_in + 1;
   __shared__ PairParamD sp[MULTI ? kMaxPairTypes : 1];
   if (MULTI) {
@@ -1010,22 +948,13 @@ __global__ __launch_bounds__(256) void k_force_fp64_piped(ForceArgs a) {
                             disp(pj.z, pi.z, qz));
     const bool in = v && (d2f < rc2);
     if (MULTI) P = sp[ti + (int)(pj.w & 0xffu)];
-    const double dx = (double)(int32_t)(pj.x - pi.x) * qdx + ((double)q.r.x - (double)ri.x);
-    const double dy = (double)(int32_t)(pj.y - pi.y) * qdy + ((double)q.r.y - (double)ri.y);
-    const double dz = (double)(int32_t)(pj.z - pi.z) * qdz + ((double)q.r.z - (double)ri.z);
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    const double ri2 = in ? 1.0 / d2 : 0.0;
-    const double ri6 = ri2 * ri2 * ri2;
-    const double fs = ri2 * ri6 * (P.B6 - P.A12 * ri6);
-    fx += fs * dx;
-    fy += fs * dy;
-    fz += fs * dz;
-    if (STATS) {
-      e += in ? ri6 * (P.A * ri6 - P.B) + P.shift : 0.0;
-      wx += fs * dx * dx;
-      wy += fs * dy * dy;
-      wz += fs * dz * dz;
-    }
+    const double dx = __builtin_fma((double)(int32_t)(pj.x - pi.x), qdx,
+                                     (double)q.r.x - (double)ri.x);
+    const double dy = __builtin_fma((double)(int32_t)(pj.y - pi.y), qdy,
+                                     (double)q.r.y - (double)ri.y);
+    const double dz = __builtin_fma((double)(int32_t)(pj.z - pi.z), qdz,
+                                     (double)q.r.z - (double)ri.z);
+    pair_fp64<STATS>(dx, dy, dz, in, P, fx, fy, fz, e, wx, wy, wz);
   };
   int ja = row(0), jb = row(1);
   asm volatile("" ::: "memory");
@@ -1098,23 +1027,13 @@ static void launch_mixed_s(int grid, int block, bool multi, const ForceArgs &a,
 }
 
 template <int T, bool STATS, bool TAIL, bool MULTI>
-static void launch_fp64_n(int grid, int block, bool piped, const ForceArgs &a,
-                          hipStream_t st) {
-  if (piped) {
-    if (a.next.active)
-      hipLaunchKernelGGL((k_force_fp64_piped<T, STATS, TAIL, MULTI, true>), dim3(grid),
-                         dim3(block), 0, st, a);
-    else
-      hipLaunchKernelGGL((k_force_fp64_piped<T, STATS, TAIL, MULTI, false>), dim3(grid),
-                         dim3(block), 0, st, a);
-  } else {
-    if (a.next.active)
-      hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, true>), dim3(grid),
-                         dim3(block), 0, st, a);
-    else
-      hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, false>), dim3(grid),
-                         dim3(block), 0, st, a);
-  }
+static void launch_fp64_n(int grid, int block, const ForceArgs &a, hipStream_t st) {
+  if (a.next.active)
+    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, true>), dim3(grid), dim3(block), 0,
+                       st, a);
+  else
+    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, false>), dim3(grid), dim3(block), 0,
+                       st, a);
 }
 
 // the energy shift only enters the statistics
@@ -1142,9 +1061,9 @@ static void launch_force_t(int precision, int unroll, int block,
     if (unroll == 1) launch_mixed_u<T, 1, STATS, TAIL>(grid, block, multi, a, st);
     else if (unroll == 2) launch_mixed_u<T, 2, STATS, TAIL>(grid, block, multi, a, st);
     else launch_mixed_u<T, 4, STATS, TAIL>(grid, block, multi, a, st);
-  } else {   // unroll 1: the FP64 form in the pipelined structure
-    if (multi) launch_fp64_n<T, STATS, TAIL, true>(grid, block, unroll == 1, a, st);
-    else launch_fp64_n<T, STATS, TAIL, false>(grid, block, unroll == 1, a, st);
+  } else {
+    if (multi) launch_fp64_n<T, STATS, TAIL, true>(grid, block, a, st);
+    else launch_fp64_n<T, STATS, TAIL, false>(grid, block, a, st);
   }
 }
 
