@@ -138,7 +138,8 @@ struct sre_engine {
   // [0] longest list, [1] total length, [2] low word: max displacement^2
   unsigned long long *d_counters = nullptr;
   uint64_t *h_info = nullptr;               // pinned readback (4 words)
-  double *h_stats = nullptr;                // pinned: 4 per replica + the force-range flag
+  double *h_stats = nullptr;                // mapped host memory: 4 per replica
+  double *m_stats = nullptr;                // its device address
   size_t h_stats_cap = 0;
   // rebuild log: every launch of the captured rebuild writes its (longest,
   // total, displacement^2 bits) to entry (launch number % kRebuildLog) of
@@ -157,12 +158,16 @@ struct sre_engine {
   // outputs
   int64_t *d_fx = nullptr, *d_fy = nullptr, *d_fz = nullptr;
   double *d_fxd = nullptr, *d_fyd = nullptr, *d_fzd = nullptr;
-  double *d_stats = nullptr;       // per replica (E, Wxx, Wyy, Wzz)
   double *d_stat_part = nullptr;   // per replica and chunk, 4 partial sums
+  unsigned *d_stat_ticket = nullptr;  // per replica: chunks summed so far
+  int stat_chunk = 0, stat_max = 0;   // atoms per chunk, of the largest replica
   unsigned long long *d_nin = nullptr;  // per replica pairs inside rc
   double *d_atom_stats = nullptr;
   double *d_tmp_out = nullptr;
-  unsigned *d_flags = nullptr;  // [0] max displacement^2 bits, [1] error bits
+  // [0] max displacement^2 bits, [1] error bits: host memory that the kernels
+  // write, so that a check is one wait and no copy
+  volatile unsigned *h_flags = nullptr;
+  unsigned *d_flags = nullptr;  // its device address
   uint64_t *d_step_ctr = nullptr;  // perturbation step counter (graph mode)
   float pert_sigma = 0.f;
   uint64_t pert_seed = 0;
@@ -257,10 +262,11 @@ sre_engine::~sre_engine() {
   dfree(d_counters); dfree(d_fx); dfree(d_fy); dfree(d_fz); dfree(d_fxd);
   if (h_info) (void)hipHostFree(h_info);
   if (h_stats) (void)hipHostFree(h_stats);
+  if (h_flags) (void)hipHostFree(const_cast<unsigned *>(h_flags));
   if (h_log) (void)hipHostFree(h_log);
   dfree(d_log_idx);
-  dfree(d_fyd); dfree(d_fzd); dfree(d_nin); dfree(d_stats); dfree(d_stat_part);
-  dfree(d_atom_stats); dfree(d_tmp_out); dfree(d_flags); dfree(d_step_ctr);
+  dfree(d_fyd); dfree(d_fzd); dfree(d_nin); dfree(d_stat_part); dfree(d_stat_ticket);
+  dfree(d_atom_stats); dfree(d_tmp_out); dfree(d_step_ctr);
   dfree(d_anchor); dfree(d_skin_part); dfree(d_build_part); dfree(d_info_slices);
   dfree(d_pos4_alt); dfree(d_res4_alt); dfree(d_backup_s); dfree(d_anchor_s);
   dfree(d_adj); dfree(d_adj_tw);
@@ -327,8 +333,14 @@ extern "C" sre_status sre_create(sre_engine **out, const sre_options *opt) {
   e->eps.assign(e->n_types * e->n_types, 1.f);
   e->sig.assign(e->n_types * e->n_types, 1.f);
   e->shift.assign(e->n_types * e->n_types, 0.f);
-  hipError_t r = dalloc(&e->d_flags, 4);
-  if (r == hipSuccess) r = hipMemsetAsync(e->d_flags, 0, 4 * sizeof(unsigned), e->stream);
+  unsigned *flags = nullptr;
+  hipError_t r = hipHostMalloc((void **)&flags, 4 * sizeof(unsigned),
+                               hipHostMallocMapped | hipHostMallocCoherent);
+  e->h_flags = flags;
+  if (r == hipSuccess) {
+    memset(flags, 0, 4 * sizeof(unsigned));
+    r = hipHostGetDevicePointer((void **)&e->d_flags, flags, 0);
+  }
   if (r == hipSuccess) r = dalloc(&e->d_counters, 3);
   if (r == hipSuccess) r = hipMemsetAsync(e->d_counters, 0, 3 * sizeof(uint64_t), e->stream);
   if (r == hipSuccess) r = hipHostMalloc((void **)&e->h_info, 4 * sizeof(uint64_t), hipHostMallocDefault);
@@ -433,8 +445,8 @@ extern "C" sre_status sre_set_system(sre_engine *e, int n_replicas,
   dfree(e->d_res4);
   dfree(e->d_nnb); dfree(e->d_fx); dfree(e->d_fy); dfree(e->d_fz);
   dfree(e->d_fxd); dfree(e->d_fyd); dfree(e->d_fzd); dfree(e->d_atom_stats);
-  dfree(e->d_stats); dfree(e->d_nin); dfree(e->d_tmp_out); dfree(e->d_tail_atom);
-  dfree(e->d_stat_part);
+  dfree(e->d_nin); dfree(e->d_tmp_out); dfree(e->d_tail_atom);
+  dfree(e->d_stat_part); dfree(e->d_stat_ticket);
   dfree(e->d_skin_part);
   dfree(e->d_pos4_alt); dfree(e->d_res4_alt); dfree(e->d_backup_s); dfree(e->d_anchor_s);
   dfree(e->d_vel); dfree(e->d_fcall); dfree(e->d_md_part);
@@ -471,9 +483,13 @@ extern "C" sre_status sre_set_system(sre_engine *e, int n_replicas,
     HIP_TRY(dalloc(&e->d_fzd, N));
   }
   HIP_TRY(dalloc(&e->d_atom_stats, (size_t)4 * N));
-  HIP_TRY(dalloc(&e->d_stats, (size_t)4 * n_replicas));
   HIP_TRY(dalloc(&e->d_nin, n_replicas));
-  HIP_TRY(dalloc(&e->d_stat_part, (size_t)4 * kStatBlocks * n_replicas));
+  e->stat_max = *std::max_element(n_atoms, n_atoms + n_replicas);
+  e->stat_chunk = stat_chunk(N);
+  HIP_TRY(dalloc(&e->d_stat_part,
+                 (size_t)4 * ((e->stat_max + e->stat_chunk - 1) / e->stat_chunk) * n_replicas));
+  HIP_TRY(dalloc(&e->d_stat_ticket, n_replicas));
+  launch_fill_u32(e->d_stat_ticket, 0u, n_replicas, e->stream);
   HIP_TRY(dalloc(&e->d_tmp_out, (size_t)4 * N));
   HIP_TRY(dalloc(&e->sb.key_a, N));
   HIP_TRY(dalloc(&e->sb.val_a, N));
@@ -1100,6 +1116,15 @@ extern "C" sre_status sre_rebuild(sre_engine *e) {
   return do_rebuild(e);
 }
 
+// The largest displacement^2 that the last launch_rebuild_info into d_flags
+// found, after the stream has been waited for.
+static float skin_disp2(const sre_engine *e) {
+  const unsigned bits = e->h_flags[0];
+  float d2;
+  memcpy(&d2, &bits, sizeof d2);
+  return d2;
+}
+
 extern "C" sre_status sre_update_positions(sre_engine *e, int *need_rebuild) {
   if (!e) return fail(SRE_ERR_INVALID, "null engine");
   if (!e->built) return fail(SRE_ERR_NOT_READY, "update before the first rebuild");
@@ -1113,12 +1138,9 @@ extern "C" sre_status sre_update_positions(sre_engine *e, int *need_rebuild) {
     launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms),
                         e->d_skin_part, 0, e->d_flags, e->stream, nullptr, nullptr, 0,
                         e->d_info_slices);
-    unsigned bits = 0;
-    HIP_TRY(hipMemcpyAsync(&bits, e->d_flags, sizeof(unsigned),
-                           hipMemcpyDeviceToHost, e->stream));
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(e->stream));
-    float d2;
-    memcpy(&d2, &bits, sizeof d2);
+    const float d2 = skin_disp2(e);
     const float half = 0.5f * e->skin;
     *need_rebuild = d2 > half * half ? 1 : 0;
   }
@@ -1194,11 +1216,21 @@ static sre_status launch_compute(sre_engine *e, unsigned flags,
 }
 
 // Reduces the per-atom statistics of the last SRE_STATS compute into
-// d_stats (stream-ordered; fixed order, so the result is reproducible).
+// h_stats (stream-ordered; fixed order, so the result is reproducible).
 static sre_status reduce_stats(sre_engine *e) {
   if (e->stats_pending) {
-    launch_stats_reduce(e->n_rep, e->d_reps, e->d_atom_stats, e->d_stat_part,
-                        e->d_stats, e->stream);
+    const size_t m = (size_t)4 * e->n_rep;
+    if (e->h_stats_cap < m) {
+      if (e->h_stats) HIP_TRY(hipHostFree(e->h_stats));
+      e->h_stats = nullptr;
+      e->h_stats_cap = 0;
+      HIP_TRY(hipHostMalloc((void **)&e->h_stats, sizeof(double) * m,
+                            hipHostMallocMapped | hipHostMallocCoherent));
+      HIP_TRY(hipHostGetDevicePointer((void **)&e->m_stats, e->h_stats, 0));
+      e->h_stats_cap = m;
+    }
+    launch_stats_reduce(e->n_rep, e->stat_max, e->stat_chunk, e->d_reps, e->d_atom_stats,
+                        e->d_stat_part, e->d_stat_ticket, e->m_stats, e->stream);
     HIP_TRY(hipGetLastError());
     e->stats_pending = false;
   }
@@ -1236,11 +1268,8 @@ extern "C" sre_status sre_step(sre_engine *e, unsigned flags, int *rebuilt) {
 // ---------------------------------------------------------------- results --
 
 static sre_status check_errors(sre_engine *e) {
-  unsigned f = 0;
-  HIP_TRY(hipMemcpyAsync(&f, e->d_flags + 1, sizeof(unsigned),
-                         hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(hipStreamSynchronize(e->stream));
-  if (f & 1u) return report_force_range(e);
+  if (e->h_flags[1] & 1u) return report_force_range(e);
   return SRE_OK;
 }
 
@@ -1296,23 +1325,10 @@ extern "C" sre_status sre_get_stats(sre_engine *e, double *out) {
   HIP_TRY(hipSetDevice(e->device));
   sre_status rs = reduce_stats(e);
   if (rs != SRE_OK) return rs;
-  // the totals and the force-range flag into pinned memory, one synchronisation
-  const size_t m = (size_t)4 * e->n_rep;
-  if (e->h_stats_cap < m + 1) {
-    if (e->h_stats) HIP_TRY(hipHostFree(e->h_stats));
-    e->h_stats = nullptr;
-    e->h_stats_cap = 0;
-    HIP_TRY(hipHostMalloc((void **)&e->h_stats, sizeof(double) * (m + 1), hipHostMallocDefault));
-    e->h_stats_cap = m + 1;
-  }
-  unsigned *flag = reinterpret_cast<unsigned *>(e->h_stats + m);
-  HIP_TRY(hipMemcpyAsync(e->h_stats, e->d_stats, sizeof(double) * m,
-                         hipMemcpyDeviceToHost, e->stream));
-  HIP_TRY(hipMemcpyAsync(flag, e->d_flags + 1, sizeof(unsigned), hipMemcpyDeviceToHost,
-                         e->stream));
+  // the totals and the force-range flag are in host memory by then
   HIP_TRY(hipStreamSynchronize(e->stream));
-  memcpy(out, e->h_stats, sizeof(double) * m);
-  if (*flag & 1u) return report_force_range(e);
+  memcpy(out, e->h_stats, sizeof(double) * 4 * e->n_rep);
+  if (e->h_flags[1] & 1u) return report_force_range(e);
   return SRE_OK;
 }
 
@@ -2186,12 +2202,9 @@ extern "C" sre_status sre_check_skin_flag(sre_engine *e) {
   launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms),
                       e->d_skin_part, 0, e->d_flags, e->stream, nullptr, nullptr, 0,
                       e->d_info_slices);
-  unsigned bits = 0;
-  HIP_TRY(hipMemcpyAsync(&bits, e->d_flags, sizeof(unsigned),
-                         hipMemcpyDeviceToHost, e->stream));
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(e->stream));
-  float d2;
-  memcpy(&d2, &bits, sizeof d2);
+  const float d2 = skin_disp2(e);
   const float half = 0.5f * e->skin;
   if (d2 > half * half)
     return fail(SRE_ERR_SKIN, "max displacement %g exceeds skin/2 = %g",
@@ -2427,16 +2440,13 @@ static sre_status md_skin_ok(sre_engine *e, bool *ok, float *disp2 = nullptr) {
   launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms),
                       e->d_skin_part, 0, e->d_flags, e->stream, nullptr, nullptr, 0,
                       e->d_info_slices);
-  unsigned bits[2] = {0, 0};
-  HIP_TRY(hipMemcpyAsync(bits, e->d_flags, 2 * sizeof(unsigned),
-                         hipMemcpyDeviceToHost, e->stream));
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(e->stream));
-  float d2;
-  memcpy(&d2, &bits[0], sizeof d2);
+  const float d2 = skin_disp2(e);
   const float half = 0.5f * e->skin;
   *ok = !(d2 > half * half);
   if (disp2) *disp2 = d2;
-  if (*ok && (bits[1] & 1u)) return report_force_range(e);
+  if (*ok && (e->h_flags[1] & 1u)) return report_force_range(e);
   return SRE_OK;
 }
 

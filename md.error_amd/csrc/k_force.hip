@@ -368,6 +368,13 @@ void launch_rebuild_info(int n_build, const int2 *build_part,
                      skin_bits, log, log_idx, log_cap);
 }
 
+// Sets the force-range flag (bit 0; no kernel sets another), which may live
+// in host memory: a store, where an atomic OR would need the host bus to know
+// one.
+__device__ __forceinline__ void raise_flag(unsigned *flag) {
+  __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------ wave reductions --
 
 template <typename V>
@@ -566,7 +573,7 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *
   // rounding of sum |fs|
   if (__ballot(act && fsabs * rc >= 1125899906842624.0f) &&
       lane == 0)
-    atomicOr(a.err_flag, 1u);
+    raise_flag(a.err_flag);
   double E = 0.0, Wx = 0.0, Wy = 0.0, Wz = 0.0;
   if (STATS) {
     E = SPLIT_E ? group_sum(-((double)wx + (double)wy + (double)wz) * (kFixInv / 12.0) -
@@ -783,7 +790,7 @@ __global__ __launch_bounds__(kWave) void k_force_cells(ForceArgs a, CellWindow c
   int64_t Fy = group_sum(__double_as_longlong(ay) - acc0, T);
   int64_t Fz = group_sum(__double_as_longlong(az) - acc0, T);
   if (__ballot(act && fsabs * rc >= 1125899906842624.0f) && lane == 0)
-    atomicOr(a.err_flag, 1u);
+    raise_flag(a.err_flag);
   double E = 0.0, Wx = 0.0, Wy = 0.0, Wz = 0.0;
   if (STATS) {
     E = SPLIT_E ? group_sum(-((double)wx + (double)wy + (double)wz) * (kFixInv / 12.0) -
@@ -1093,18 +1100,27 @@ void launch_force(int precision, int lanes, int unroll, int block, bool stats,
 
 // ------------------------------------------------------ statistic reduce --
 
-// Replica sums of the per-atom (E, Wxx, Wyy, Wzz) in a fixed order: block
-// (b, r) sums the b-th of kStatBlocks contiguous chunks of replica r's atoms
-// (contiguous in sorted order; thread k takes atoms k, k + 256, ... of the
-// chunk, then a fixed shuffle tree and LDS pass); k_stats_final adds the
-// chunks in order.
-__global__ __launch_bounds__(256) void k_stats_partial(const RepInfo *reps,
-                                                       const double *atom_stats,
-                                                       double *part) {
+// Replica sums of the per-atom (E, Wxx, Wyy, Wzz) in a fixed order, one launch:
+// block (b, r) sums the b-th chunk of replica r's atoms (contiguous in sorted
+// order; thread k takes atoms k, k + 256, ... of the chunk, then a fixed
+// shuffle tree and LDS pass); the last of the replica's blocks to finish adds
+// the chunks' sums, in a fixed tree too, and writes the totals where the host
+// reads them (or to device memory).  The chunks' sums pass between XCDs, whose
+// L2 caches do not see each other's lines: they are stored and loaded at agent
+// scope.  What bounds it: latency (one round of loads, the ticket, the host
+// write); at 2 million atoms the 64 MB it reads.  As two launches, of 32 chunks
+// per replica and of the totals, with a copy each of totals and flag, a step
+// of 64 000 atoms in FP64 with its statistics took 46.2 us, now 42.2; the sums
+// of 2 million atoms took 122 us, now 27.
+__global__ __launch_bounds__(256) void k_stats_reduce(int chunk, const RepInfo *reps,
+                                                      const double *atom_stats, double *part,
+                                                      unsigned *ticket, double *stats) {
   __shared__ double red[256 / kWave][4];
+  __shared__ bool last;
   const int b = blockIdx.x, r = blockIdx.y;
   const RepInfo &R = reps[r];
-  const int chunk = (R.n_atoms + kStatBlocks - 1) / kStatBlocks;
+  const int nb = (R.n_atoms + chunk - 1) / chunk;     // the replica's chunks
+  if (b >= nb) return;
   const int i0 = b * chunk, i1 = min(R.n_atoms, i0 + chunk);
   double acc[4] = {0, 0, 0, 0};
   for (int i = i0 + (int)threadIdx.x; i < i1; i += blockDim.x) {
@@ -1118,30 +1134,52 @@ __global__ __launch_bounds__(256) void k_stats_partial(const RepInfo *reps,
   if ((threadIdx.x & (kWave - 1)) == 0)
     for (int c = 0; c < 4; ++c) red[wv][c] = acc[c];
   __syncthreads();
+  part += (size_t)r * gridDim.x * 4;
   if (threadIdx.x == 0) {
     for (int k = 1; k < (int)(blockDim.x / kWave); ++k)
       for (int c = 0; c < 4; ++c) acc[c] += red[k][c];
-    for (int c = 0; c < 4; ++c) part[((size_t)r * kStatBlocks + b) * 4 + c] = acc[c];
+    if (nb == 1)
+      for (int c = 0; c < 4; ++c) stats[4 * r + c] = acc[c];
+    for (int c = 0; c < 4 && nb > 1; ++c)
+      __hip_atomic_store(part + (size_t)b * 4 + c, acc[c], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    // the four stores have arrived before the ticket is drawn (a release would
+    // also write back the XCD's whole L2, the forces just computed with it:
+    // 44 us more with 64 replicas)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = nb > 1 && __hip_atomic_fetch_add(ticket + r, 1u, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nb - 1u;
+    asm volatile("" ::: "memory");
   }
+  __syncthreads();
+  if (!last || threadIdx.x >= kWave) return;
+  // one wavefront: component lane % 4 of chunks lane / 4, + 16, ...
+  const int lane = threadIdx.x, c = lane & 3;
+  double t = 0.0;
+  for (int k = lane >> 2; k < nb; k += kWave / 4)
+    t += __hip_atomic_load(part + (size_t)k * 4 + c, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int o = 4; o < kWave; o <<= 1) t += __shfl_xor(t, o, kWave);
+  if (lane < 4) stats[4 * r + c] = t;
+  if (lane == 0) ticket[r] = 0u;
 }
 
-__global__ __launch_bounds__(256) void k_stats_final(int n_rep, const double *part,
-                                                     double *stats) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // (replica, component)
-  if (t >= 4 * n_rep) return;
-  const int r = t / 4, c = t % 4;
-  double acc = 0.0;
-  for (int b = 0; b < kStatBlocks; ++b) acc += part[((size_t)r * kStatBlocks + b) * 4 + c];
-  stats[t] = acc;
+// 1 024 atoms per chunk (62 500 atoms: 6.4 us, with 2 048 7.1, with 8 000
+// 13.8), but no more than some 512 chunks: the tickets of one line of memory
+// follow each other every 10 ns (2 million atoms: 27 us with 512 chunks, 38
+// with 1 024; 64 replicas of 0.7 million atoms in all: 10 with 512, 38 with
+// 4 096)
+int stat_chunk(int n) {
+  const int c = (n + 511) / 512;
+  return c > 1024 ? c : 1024;
 }
 
-void launch_stats_reduce(int n_rep, const RepInfo *reps,
-                         const double *atom_stats, double *part, double *stats,
-                         hipStream_t st) {
-  hipLaunchKernelGGL(k_stats_partial, dim3(kStatBlocks, n_rep), dim3(256), 0, st,
-                     reps, atom_stats, part);
-  hipLaunchKernelGGL(k_stats_final, dim3((4 * n_rep + 255) / 256), dim3(256), 0,
-                     st, n_rep, part, stats);
+void launch_stats_reduce(int n_rep, int n_max, int chunk, const RepInfo *reps,
+                         const double *atom_stats, double *part, unsigned *ticket,
+                         double *stats, hipStream_t st) {
+  hipLaunchKernelGGL(k_stats_reduce, dim3((n_max + chunk - 1) / chunk, n_rep), dim3(256), 0,
+                     st, chunk, reps, atom_stats, part, ticket, stats);
 }
 
 // Pairs of the list inside the cutoff (d^2 < rc_i^2, the force kernel's

@@ -586,12 +586,15 @@ void launch_force(int precision, int lanes, int unroll, int block, bool stats,
                   bool tail,
                   const ForceArgs &a, hipStream_t st);
 int force_num_waves(int n, int lanes);
-// stats[4 r + c] = sum over replica r's atoms of atom_stats[4 s + c];
-// part holds n_rep * kStatBlocks * 4 doubles of chunk partials
-constexpr int kStatBlocks = 32;
-void launch_stats_reduce(int n_rep, const RepInfo *reps,
-                         const double *atom_stats, double *part, double *stats,
-                         hipStream_t st);
+// stats[4 r + c] = sum over replica r's atoms of atom_stats[4 s + c], in chunks
+// of `chunk` atoms (stat_chunk of all atoms, or more); n_max is the largest
+// replica's size, part holds 4 doubles per replica and chunk of that one,
+// ticket n_rep words that are zero before the first launch and after each.
+// stats may be mapped host memory.
+int stat_chunk(int n);
+void launch_stats_reduce(int n_rep, int n_max, int chunk, const RepInfo *reps,
+                         const double *atom_stats, double *part, unsigned *ticket,
+                         double *stats, hipStream_t st);
 // counts[r] += pairs of replica r's lists with d^2 < rc_i^2 (counts zeroed
 // by the caller)
 void launch_count_in_rc(int n, int lanes, int cap, const uint4 *pos4,

@@ -10,6 +10,7 @@
 // on a device is looked up once (hipGetSymbolAddress) and only that address
 // is handed to kernels and copies.  Every call on a GPU shares that GPU's
 // array, so calls that overlap on one GPU race.
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -19,6 +20,7 @@
 namespace sre {
 
 constexpr size_t kScratchBytes = (size_t)40 << 20;   // 40 MiB per GPU
+constexpr int kStatChunks = 32;      // at most, of the statistics reduction
 constexpr int kStaticMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -181,9 +183,10 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   int64_t *d_fy = c.take<int64_t>(N);
   int64_t *d_fz = c.take<int64_t>(N);
   double *d_atom_stats = c.take<double>((size_t)4 * N);
-  double *d_stat_part = c.take<double>((size_t)4 * kStatBlocks);
-  double *d_stats = c.take<double>(4);
-  unsigned *d_flags = c.take<unsigned>(4);
+  double *d_stat_part = c.take<double>((size_t)4 * kStatChunks);
+  // totals, then the flags (one copy back) and the reduction's ticket
+  double *d_stats = c.take<double>(6);
+  unsigned *d_flags = reinterpret_cast<unsigned *>(d_stats + 4);
   if (!c.fits())
     return fail(SRE_ERR_INVALID,
                 "sre_forces_static: the system needs %zu bytes of scratch (limit %zu; "
@@ -243,13 +246,14 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   launch_force(SRE_PREC_MIXED, T, U, block, true, false, a, st);
   launch_export_forces(N, sb.val_a, d_fx, d_fy, d_fz, nullptr, nullptr, nullptr, d_forces,
                        nullptr, st);
-  launch_stats_reduce(1, d_reps, d_atom_stats, d_stat_part, d_stats, st);
+  launch_stats_reduce(1, N, std::max(stat_chunk(N), (N + kStatChunks - 1) / kStatChunks), d_reps, d_atom_stats, d_stat_part, d_flags + 2,
+                      d_stats, st);
   HIP_TRY(hipGetLastError());
-  double host_stats[4];
-  unsigned flags[2] = {0, 0};
+  double host_stats[5];
   HIP_TRY(hipMemcpyAsync(host_stats, d_stats, sizeof host_stats, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(flags, d_flags, sizeof flags, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
+  unsigned flags[2];
+  memcpy(flags, host_stats + 4, sizeof flags);
   if (flags[1] & 1u)
     return fail(SRE_ERR_FORCE_RANGE,
                 "pair forces beyond the exact fixed-point range (overlapping atoms?)");
