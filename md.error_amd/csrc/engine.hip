@@ -229,7 +229,7 @@ struct sre_engine {
   float *d_vel = nullptr;          // 3 per atom
   float *d_fcall = nullptr;        // force of the last kick, 3 per atom
   double *d_md_part = nullptr;     // kick partial sums (K, Px, Py, Pz) per block
-  MDState *d_md = nullptr;
+  MDState *d_md = nullptr, *d_md_next = nullptr;   // d_md_next: between drift and kick
   MDState md{};                    // host copy of the parameters
   bool vel_set = false, md_set = false;
   int md_since_rebuild = 0;        // MD steps since the last rebuild
@@ -270,7 +270,7 @@ sre_engine::~sre_engine() {
   dfree(d_anchor); dfree(d_skin_part); dfree(d_build_part); dfree(d_info_slices);
   dfree(d_pos4_alt); dfree(d_res4_alt); dfree(d_backup_s); dfree(d_anchor_s);
   dfree(d_adj); dfree(d_adj_tw);
-  dfree(d_mass); dfree(d_vel); dfree(d_fcall); dfree(d_md_part); dfree(d_md);
+  dfree(d_mass); dfree(d_vel); dfree(d_fcall); dfree(d_md_part); dfree(d_md); dfree(d_md_next);
   dfree(d_fc);
   dfree(d_snap_pos); dfree(d_snap_vel); dfree(d_snap_fcall); dfree(d_snap_part);
   dfree(d_snap_md);
@@ -1131,7 +1131,7 @@ extern "C" sre_status sre_update_positions(sre_engine *e, int *need_rebuild) {
   HIP_TRY(hipSetDevice(e->device));
   launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
                           e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
-                          e->d_res4, e->d_skin_part, nullptr, nullptr, e->stream);
+                          e->d_res4, e->d_skin_part, nullptr, e->stream);
   HIP_TRY(hipGetLastError());
   e->stats_valid = e->forces_valid = e->atom_stats_valid = false;
   if (need_rebuild) {
@@ -1812,26 +1812,33 @@ extern "C" sre_status sre_autotune(sre_engine *e, unsigned flags,
 
 // MD step pieces (k_md.hip): the factors of the step from the last kick's
 // sums, then kick + drift + refresh, and after the force the second kick
-static void enqueue_md_drift(sre_engine *e) {
-  launch_md_factors(e->n_atoms, e->d_md_part, e->d_md, e->stream);
-  DriftArgs d{e->d_vel, e->d_fcall, e->d_mass, e->d_types, e->d_md,
-              (float)e->md.dt};
-  launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
-                          e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
-                          e->d_res4, e->d_skin_part, nullptr, &d, e->stream);
+// d_md_next where the drift computes the factors itself, else NULL
+static MDState *md_next(const sre_engine *e) {
+  return md_fold_factors(e->n_atoms) ? e->d_md_next : nullptr;
 }
 
-static void enqueue_md_kick(sre_engine *e, float hdt) {
+static void enqueue_md_drift(sre_engine *e) {
+  DriftArgs d{e->d_vel, e->d_fcall, e->d_mass, e->d_types, e->d_md_part, e->d_md,
+              md_next(e), (float)e->md.dt};
+  launch_md_drift(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
+                  e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
+                  e->d_res4, e->d_skin_part, d, e->stream);
+}
+
+// after_drift: the kick that ends a step, which also stores the state that
+// the step's drift advanced
+static void enqueue_md_kick(sre_engine *e, float hdt, bool after_drift) {
   launch_md_kick(e->n_atoms, e->d_inv_perm, e->d_types, e->d_fx, e->d_fy,
                  e->d_fz, e->d_fxd, e->d_fyd, e->d_fzd, e->d_mass, hdt,
-                 e->d_vel, e->d_fcall, e->d_md_part, e->stream);
+                 e->d_vel, e->d_fcall, e->d_md_part, e->d_md,
+                 after_drift ? md_next(e) : nullptr, e->stream);
 }
 
 static sre_status enqueue_md_step(sre_engine *e, unsigned flags) {
   enqueue_md_drift(e);
   sre_status s = launch_compute(e, flags & (SRE_STATS | SRE_TAIL | SRE_FCORR), nullptr);
   if (s != SRE_OK) return s;
-  enqueue_md_kick(e, (float)(0.5 * e->md.dt));
+  enqueue_md_kick(e, (float)(0.5 * e->md.dt), true);
   return SRE_OK;
 }
 
@@ -1857,7 +1864,7 @@ static sre_status enqueue_fused_steps(sre_engine *e, unsigned flags, int K,
   auto res4_of = [&](int j) { return ((K - 1 - j) % 2 == 0) ? e->d_res4 : e->d_res4_alt; };
   launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
                           e->pos_stride, e->d_reps, rep0(e), pos4_of(0), e->d_backup,
-                          res4_of(0), e->d_skin_part, &pa, nullptr, e->stream);
+                          res4_of(0), e->d_skin_part, &pa, e->stream);
   refresh_tail_values(e);
   NextRefresh nx{};
   nx.active = 1;
@@ -1931,8 +1938,7 @@ static sre_status enqueue_steps(sre_engine *e, unsigned flags, int K,
     }
     launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
                             e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
-                            e->d_res4, e->d_skin_part, pert ? &pa : nullptr, nullptr,
-                            e->stream);
+                            e->d_res4, e->d_skin_part, pert ? &pa : nullptr, e->stream);
     s = launch_compute(e, flags & (SRE_STATS | SRE_TAIL | SRE_FCORR),
                        pert ? e->d_step_ctr : nullptr);
   }
@@ -2278,6 +2284,7 @@ static sre_status md_buffers(sre_engine *e) {
   }
   if (!e->d_md) {
     HIP_TRY(dalloc(&e->d_md, 1));
+    HIP_TRY(dalloc(&e->d_md_next, 1));
     HIP_TRY(dalloc(&e->d_mass, kMaxTypes));
     e->graph_epoch++;
   }
@@ -2506,7 +2513,7 @@ extern "C" sre_status sre_md_run(sre_engine *e, int n_steps, int rebuild_every,
     launch_update_positions(e->n_atoms, e->d_inv_perm,
                             const_cast<float *>(e->d_pos), e->pos_stride,
                             e->d_reps, rep0(e), e->d_pos4, e->d_backup, e->d_res4,
-                            e->d_skin_part, nullptr, nullptr, e->stream);
+                            e->d_skin_part, nullptr, e->stream);
     HIP_TRY(hipGetLastError());
     bool ok;
     s = md_skin_ok(e, &ok);
@@ -2524,7 +2531,7 @@ extern "C" sre_status sre_md_run(sre_engine *e, int n_steps, int rebuild_every,
   // caller order and leaves the kinetic energy and momentum sums
   s = launch_compute(e, fl);
   if (s != SRE_OK) return s;
-  enqueue_md_kick(e, 0.f);
+  enqueue_md_kick(e, 0.f, false);
   HIP_TRY(hipGetLastError());
   if (n_steps == 0) {
     launch_md_finish(e->n_atoms, e->d_md_part, e->d_md, e->d_vel, e->stream);
@@ -2603,16 +2610,18 @@ extern "C" sre_status sre_md_run(sre_engine *e, int n_steps, int rebuild_every,
       HIP_TRY(hipGetLastError());
       bool ok;
       s = md_skin_ok(e, &ok);
-      if (s != SRE_OK) return s;
-      if (!ok) {
+      if (s == SRE_OK && !ok) {
         // (a range flag raised before this point is seen by the next check)
         s = do_rebuild(e);
-        if (s != SRE_OK) return s;
-        if (n_rebuilds) ++*n_rebuilds;
+        if (s == SRE_OK && n_rebuilds) ++*n_rebuilds;
       }
-      s = launch_compute(e, left == 1 ? flags : fl);
-      if (s != SRE_OK) return s;
-      enqueue_md_kick(e, (float)(0.5 * e->md.dt));
+      if (s == SRE_OK) s = launch_compute(e, left == 1 ? flags : fl);
+      if (s != SRE_OK) {
+        // a step left half done keeps the state that its drift advanced
+        if (md_next(e)) launch_md_store(e->d_md, e->d_md_next, e->stream);
+        return s;
+      }
+      enqueue_md_kick(e, (float)(0.5 * e->md.dt), true);
       HIP_TRY(hipGetLastError());
       ++e->md_since_rebuild;
       --left;

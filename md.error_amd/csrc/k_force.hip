@@ -24,22 +24,6 @@ namespace sre {
 // inv_perm[i].  The skin test compares with the rebuild-time lattice position
 // backup[i]; each wavefront keeps the largest squared displacement it has
 // seen since the last rebuild in its own slot of skin_part (no atomics).
-// With drift.vel set the refresh is the first half of a velocity Verlet step
-// (H/src/Integrator.cu:273-324, velocityVerlet_part1) after the thermostat
-// and centre-of-mass factors of the step: v <- a2 (a1 v - vcom) + F dt/(2m),
-// x <- x + v dt, then x is wrapped back into [0, L) by one add or subtract of
-// L (the reference wraps at each rebuild, H/src/MDSystem_interface.cu:19-36).
-__device__ __forceinline__ Geom geom_of(const RepInfo &R) {
-  Geom g;
-  for (int d = 0; d < 3; ++d) {
-    g.L[d] = R.L[d];
-    g.q[d] = R.q[d];
-    g.invq[d] = R.invq[d];
-    g.qd[d] = R.qd[d];
-  }
-  return g;
-}
-
 // Every load an atom needs is issued before any of them is used (the
 // refresh runs one wavefront per SIMD at 64k atoms, so the memory round trip
 // is its cost); with one replica the geometry comes in the kernel arguments.
@@ -47,8 +31,7 @@ __global__ __launch_bounds__(256) void k_update_positions(
     int n, const uint32_t *__restrict__ inv_perm, float *__restrict__ pos,
     int stride, const RepInfo *__restrict__ reps, Geom g1, int one_rep,
     uint4 *__restrict__ pos4, const uint4 *__restrict__ backup,
-    float4 *__restrict__ res4, float *__restrict__ skin_part, PerturbArgs pert,
-    DriftArgs drift) {
+    float4 *__restrict__ res4, float *__restrict__ skin_part, PerturbArgs pert) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int w = i / kWave;  // slots exist for the waves holding atoms
   const bool wslot = w * kWave < n;
@@ -60,7 +43,6 @@ __global__ __launch_bounds__(256) void k_update_positions(
     const uint32_t s = inv_perm[i];
     float *p = pos + (size_t)i * stride;
     float x, y, z;
-    bool wrap = false;
     if (pert.step_ctr) {
       const float *o = pert.anchor ? pert.anchor + (size_t)i * stride : p;
       const float ox = o[0], oy = o[1], oz = o[2];
@@ -71,26 +53,6 @@ __global__ __launch_bounds__(256) void k_update_positions(
       p[0] = x;
       p[1] = y;
       p[2] = z;
-    } else if (drift.vel) {
-      float *v = drift.vel + (size_t)i * 3;
-      const float *f = drift.fcall + (size_t)i * 3;
-      const float v0 = v[0], v1 = v[1], v2 = v[2];
-      const float f0 = f[0], f1 = f[1], f2 = f[2];
-      const float p0 = p[0], p1 = p[1], p2 = p[2];
-      const float m = drift.mass[drift.types[i]];
-      const MDState &ms = *drift.state;
-      const float a1 = (float)ms.a1, a2 = (float)ms.a2;
-      const float c = 0.5f * drift.dt / m;
-      const float vx = a2 * (a1 * v0 - (float)ms.vcom[0]) + c * f0;
-      const float vy = a2 * (a1 * v1 - (float)ms.vcom[1]) + c * f1;
-      const float vz = a2 * (a1 * v2 - (float)ms.vcom[2]) + c * f2;
-      v[0] = vx;
-      v[1] = vy;
-      v[2] = vz;
-      x = p0 + vx * drift.dt;
-      y = p1 + vy * drift.dt;
-      z = p2 + vz * drift.dt;
-      wrap = true;
     } else {
       x = p[0];
       y = p[1];
@@ -98,16 +60,6 @@ __global__ __launch_bounds__(256) void k_update_positions(
     }
     // R: the atom's replica; with one replica its geometry is an argument
     const Geom G = one_rep ? g1 : geom_of(reps[b.w >> 8]);
-    if (wrap) {
-      // x + v dt wrapped back into [0, L) by one add or subtract of L (the
-      // reference wraps at each rebuild, H/src/MDSystem_interface.cu:19-36)
-      x = x < 0.f ? x + G.L[0] : (x >= G.L[0] ? x - G.L[0] : x);
-      y = y < 0.f ? y + G.L[1] : (y >= G.L[1] ? y - G.L[1] : y);
-      z = z < 0.f ? z + G.L[2] : (z >= G.L[2] ? z - G.L[2] : z);
-      p[0] = x;
-      p[1] = y;
-      p[2] = z;
-    }
     const uint32_t ux = quantize(x, G.invq[0]);
     const uint32_t uy = quantize(y, G.invq[1]);
     const uint32_t uz = quantize(z, G.invq[2]);
@@ -216,24 +168,14 @@ __device__ __forceinline__ bool force_block(const ForceArgs &a, int *bid, int *n
 void launch_update_positions(int n, const uint32_t *inv_perm, float *pos,
                              int stride, const RepInfo *reps, const RepInfo *host_rep0,
                              uint4 *pos4, const uint4 *backup, float4 *res4,
-                             float *skin_part, const PerturbArgs *pert,
-                             const DriftArgs *drift, hipStream_t st) {
+                             float *skin_part, const PerturbArgs *pert, hipStream_t st) {
   if (n <= 0) return;
   PerturbArgs p{};
   if (pert) p = *pert;
-  DriftArgs d{};
-  if (drift) d = *drift;
-  Geom g{};
-  if (host_rep0)
-    for (int k = 0; k < 3; ++k) {
-      g.L[k] = host_rep0->L[k];
-      g.q[k] = host_rep0->q[k];
-      g.invq[k] = host_rep0->invq[k];
-      g.qd[k] = host_rep0->qd[k];
-    }
+  const Geom g = host_rep0 ? geom_of(*host_rep0) : Geom{};
   hipLaunchKernelGGL(k_update_positions, dim3((n + 255) / 256), dim3(256), 0,
                      st, n, inv_perm, pos, stride, reps, g, host_rep0 ? 1 : 0, pos4,
-                     backup, res4, skin_part, p, d);
+                     backup, res4, skin_part, p);
 }
 
 // ------------------------------------------------------- rebuild info --

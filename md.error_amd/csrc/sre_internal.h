@@ -421,6 +421,16 @@ struct Geom {
   float L[3], q[3];
   double invq[3], qd[3];
 };
+__host__ __device__ inline Geom geom_of(const RepInfo &R) {
+  Geom g;
+  for (int d = 0; d < 3; ++d) {
+    g.L[d] = R.L[d];
+    g.q[d] = R.q[d];
+    g.invq[d] = R.invq[d];
+    g.qd[d] = R.qd[d];
+  }
+  return g;
+}
 
 // step_ctr (optional) is advanced by one thread after the positions are read
 // Optional perturbation folded into the position refresh:
@@ -445,15 +455,17 @@ struct MDState {
   double dt, total_mass;
   int thermostat, remove_com, have_end, pad;
 };
-// Optional velocity Verlet kick + drift folded into the position refresh:
-// v <- a2 (a1 v - vcom) + F dt / (2 m); x <- x + v dt (caller order; F from
-// fcall, saved by the previous kick).
+// Velocity Verlet kick + drift with the position refresh, after the factors of
+// the step: v <- a2 (a1 v - vcom) + F dt / (2 m); x <- x + v dt (caller order;
+// F from fcall and the sums of `part`, both of the previous kick).
 struct DriftArgs {
   float *vel;
   const float *fcall;
   const float *mass;   // per type
   const int *types;
-  const MDState *state;
+  const double *part;
+  MDState *state;      // advanced in place when next is NULL
+  MDState *next;       // or left as it is, the advanced one here
   float dt;
 };
 // Grid force correction (AssignForceCorr::assign + the force add of the
@@ -476,9 +488,15 @@ void launch_md_kick(int n, const uint32_t *inv_perm, const int *types,
                     const int64_t *fx, const int64_t *fy, const int64_t *fz,
                     const double *fxd, const double *fyd, const double *fzd,
                     const float *mass, float hdt, float *vel, float *fcall,
-                    double *part, hipStream_t st);
-void launch_md_factors(int n, const double *part, MDState *state,
-                       hipStream_t st);
+                    double *part, MDState *state, const MDState *next, hipStream_t st);
+// whether the drift computes the factors itself: it then leaves the advanced
+// state in DriftArgs::next, and the kick that follows stores it
+bool md_fold_factors(int n);
+void launch_md_store(MDState *state, const MDState *next, hipStream_t st);
+void launch_md_drift(int n, const uint32_t *inv_perm, float *pos, int stride,
+                     const RepInfo *reps, const RepInfo *host_rep0, uint4 *pos4,
+                     const uint4 *backup, float4 *res4, float *skin_part,
+                     const DriftArgs &drift, hipStream_t st);
 void launch_md_finish(int n, const double *part, MDState *state, float *vel,
                       hipStream_t st);
 // Position refresh + skin test: each wavefront keeps the largest squared
@@ -490,8 +508,7 @@ inline int skin_part_count(int n) { return (n + kWave - 1) / kWave; }
 void launch_update_positions(int n, const uint32_t *inv_perm, float *pos,
                              int stride, const RepInfo *reps, const RepInfo *host_rep0,
                              uint4 *pos4, const uint4 *backup, float4 *res4,
-                             float *skin_part, const PerturbArgs *pert,
-                             const DriftArgs *drift, hipStream_t st);
+                             float *skin_part, const PerturbArgs *pert, hipStream_t st);
 
 // The next step's position refresh folded into a force launch (perturbation
 // mode, no integrator): n_blocks blocks in front of the force blocks
