@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sre.h"
@@ -45,6 +46,8 @@ constexpr int kRebuildLog = 1024;    // rebuild-log entries (segments per queue)
 // internal step-graph flag: the K steps are MD steps (thermostat factors,
 // kick + drift refresh, force, kick) and SRE_STATS applies to the last only
 constexpr unsigned kGraphMD = 1u << 16;
+constexpr unsigned kGraphSnap = 1u << 17;     // the MD snapshot before the steps
+constexpr unsigned kGraphRebuild = 1u << 18;  // a rebuild behind them
 
 struct sre_engine {
   int device = 0;
@@ -201,8 +204,10 @@ struct sre_engine {
   size_t adj_cap = 0;
   int64_t *d_adj_tw = nullptr;
   size_t adj_tw_cap = 0;
-  // step graphs: K steps of [refresh + force] each, cached by (flags, K)
+  // step graphs: K steps of [refresh + force] each, cached by (flags, K), with
+  // a rebuild behind them also by its arguments
   struct StepGraph {
+    std::vector<unsigned char> sig;
     hipGraphExec_t exec = nullptr;
     unsigned flags = 0;
     int steps = 0;
@@ -992,7 +997,9 @@ static void enqueue_rebuild(sre_engine *e, int n_parts, hipStream_t st,
                             e->d_rep_of, e->d_reps, e->d_rc, e->n_types, e->sb,
                             e->d_cell_count, e->d_start, e->d_pos4, e->d_backup,
                             e->d_inv_perm, e->d_res4, e->d_rcut, e->d_tail_idx,
-                            rc_atom, e->d_backup_s, anchor, e->d_anchor_s, st, counted);
+                            rc_atom, e->d_backup_s, anchor, e->d_anchor_s, st,
+                            EarlySkin{e->d_skin_part, skin_part_count(N), e->d_log,
+                                      e->d_log_idx, kRebuildLog}, counted);
   } else {
     launch_radix_sort(N, e->key_bits, e->d_pos, e->pos_stride, e->d_rep_of,
                       e->d_reps, e->sb, st);
@@ -1011,17 +1018,24 @@ static void enqueue_rebuild(sre_engine *e, int n_parts, hipStream_t st,
                       st, e->d_log, e->d_log_idx, kRebuildLog, e->d_info_slices);
 }
 
-// Queues one launch of the captured rebuild; returns its rebuild-log entry
-// (valid once the stream has been synchronised).
-static hipError_t launch_rebuild(sre_engine *e, const uint64_t **entry) {
-  hipError_t r = hipGraphLaunch(e->rebuild_exec, e->stream);
+// No displacement^2: a rebuild-log word that its launch has not yet written.
+constexpr uint64_t kNotYet = ~0ull;
+
+// Queues one launch of a graph with one rebuild; returns its rebuild-log entry
+// (valid once the stream has been synchronised; its displacement from when it
+// is no longer kNotYet).
+static hipError_t launch_rebuild(sre_engine *e, hipGraphExec_t exec, const uint64_t **entry) {
+  uint64_t *dst = e->h_log + 3 * (size_t)(e->log_launches % kRebuildLog);
+  *static_cast<volatile uint64_t *>(dst + 2) = kNotYet;
+  hipError_t r = hipGraphLaunch(exec, e->stream);
   if (r != hipSuccess) return r;
-  *entry = e->h_log + 3 * (size_t)(e->log_launches % kRebuildLog);
+  *entry = dst;
   ++e->log_launches;
   return hipSuccess;
 }
 
-static sre_status do_rebuild(sre_engine *e) {
+// Everything up to the launch of the device sequence.
+static sre_status rebuild_begin(sre_engine *e, const uint64_t **info) {
   if (!e->system_set) return fail(SRE_ERR_INVALID, "rebuild: system not set");
   if (!e->types_set) return fail(SRE_ERR_INVALID, "rebuild: types not set");
   if (!e->params_set) return fail(SRE_ERR_INVALID, "rebuild: pair parameters not set");
@@ -1077,9 +1091,20 @@ static sre_status do_rebuild(sre_engine *e) {
     HIP_TRY(hipGraphUpload(e->rebuild_exec, st));
     e->rebuild_sig = std::move(sig);
   }
-  const uint64_t *info = nullptr;
-  HIP_TRY(launch_rebuild(e, &info));
-  HIP_TRY(hipStreamSynchronize(st));
+  HIP_TRY(launch_rebuild(e, e->rebuild_exec, info));
+  return SRE_OK;
+}
+
+// The capacity for lists of up to mc entries after an overflow.
+static int grown_cap(const sre_engine *e, int mc) {
+  return round_up(std::max(mc + 16, (int)(mc * 1.2)), e->tune.force_lanes);
+}
+
+// The rest, after the stream has been synchronised: the results of the log
+// entry, and larger lists if it tells of an overflow.
+static sre_status rebuild_end(sre_engine *e, const uint64_t *info) {
+  hipStream_t st = e->stream;
+  const int n_parts = build_part_count(e->tune.build_mode, e->n_atoms, e->n_cols);
   for (int k = 0; k < 3; ++k) e->h_info[k] = info[k];
   {
     const unsigned bits = (unsigned)(e->h_info[2] & 0xffffffffu);
@@ -1094,8 +1119,7 @@ static sre_status do_rebuild(sre_engine *e) {
     if (attempt == 3)
       return fail(SRE_ERR_LIST_OVERFLOW, "neighbor list overflow (%d > %d)", mc,
                   e->cap);
-    cap = round_up(std::max(mc + 16, (int)(mc * 1.2)), e->tune.force_lanes);
-    s = ensure_list(e, cap);
+    sre_status s = ensure_list(e, grown_cap(e, mc));
     if (s != SRE_OK) return s;
     enqueue_build(e, st);
     launch_rebuild_info(n_parts, e->d_build_part, e->d_counters, 0, e->d_skin_part,
@@ -1108,6 +1132,37 @@ static sre_status do_rebuild(sre_engine *e) {
   e->built = true;
   e->md_since_rebuild = 0;
   e->stats_valid = e->forces_valid = e->atom_stats_valid = false;
+  return SRE_OK;
+}
+
+static sre_status do_rebuild(sre_engine *e) {
+  const uint64_t *info = nullptr;
+  sre_status s = rebuild_begin(e, &info);
+  if (s != SRE_OK) return s;
+  HIP_TRY(hipStreamSynchronize(e->stream));
+  return rebuild_end(e, info);
+}
+
+// Waits until the queued rebuild of this log entry has written the largest
+// displacement^2 of the steps before it, which is its first launch's work.
+static sre_status wait_disp2(sre_engine *e, const uint64_t *info, float *d2) {
+  const volatile uint64_t *w = info + 2;
+  for (unsigned k = 1; *w == kNotYet; ++k) {
+    if (k % 4096 != 0) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    // the stream ends (or fails) without it: never by a rebuild's design
+    const hipError_t r = hipStreamQuery(e->stream);
+    if (r == hipErrorNotReady) {
+      std::this_thread::yield();
+      continue;
+    }
+    if (r != hipSuccess) return fail(SRE_ERR_HIP, "rebuild: %s", hipGetErrorString(r));
+    if (*w == kNotYet) return fail(SRE_ERR_HIP, "rebuild: no displacement in the log");
+  }
+  const unsigned bits = (unsigned)(*w & 0xffffffffu);
+  memcpy(d2, &bits, sizeof(float));
   return SRE_OK;
 }
 
@@ -1834,6 +1889,8 @@ static void enqueue_md_kick(sre_engine *e, float hdt, bool after_drift) {
                  after_drift ? md_next(e) : nullptr, e->stream);
 }
 
+static void enqueue_snapshot(sre_engine *e, bool restore);
+
 static sre_status enqueue_md_step(sre_engine *e, unsigned flags) {
   enqueue_md_drift(e);
   sre_status s = launch_compute(e, flags & (SRE_STATS | SRE_TAIL | SRE_FCORR), nullptr);
@@ -1948,11 +2005,14 @@ static sre_status enqueue_steps(sre_engine *e, unsigned flags, int K,
 // Captures K steps of [refresh (+ perturbation) + force] into one graph, or
 // returns the cached one; the graph reads the engine's buffers by address, so
 // every reallocation or layout change bumps graph_epoch and invalidates it.
+// kGraphRebuild: the rebuild as last prepared (rebuild_begin), whose arguments
+// must be the engine's still.
 static sre_status step_graph(sre_engine *e, unsigned flags, int K,
                              hipGraphExec_t *out) {
   sre_engine::StepGraph *slot = nullptr, *lru = &e->step_graphs[0];
   for (sre_engine::StepGraph &g : e->step_graphs) {
-    if (g.exec && g.flags == flags && g.steps == K && g.epoch == e->graph_epoch)
+    if (g.exec && g.flags == flags && g.steps == K && g.epoch == e->graph_epoch &&
+        (!(flags & kGraphRebuild) || g.sig == e->rebuild_sig))
       slot = &g;
     if (g.last_use < lru->last_use) lru = &g;
   }
@@ -1967,7 +2027,11 @@ static sre_status step_graph(sre_engine *e, unsigned flags, int K,
       return fail(SRE_ERR_INVALID, "SRE_PERTURB needs sre_set_perturbation first");
     hipGraph_t g;
     HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+    if (flags & kGraphSnap) enqueue_snapshot(e, false);
     sre_status s = enqueue_steps(e, flags, K);
+    if (s == SRE_OK && (flags & kGraphRebuild))
+      enqueue_rebuild(e, build_part_count(e->tune.build_mode, e->n_atoms, e->n_cols),
+                      e->stream);
     hipError_t r = hipStreamEndCapture(e->stream, &g);
     if (s != SRE_OK) {
       if (r == hipSuccess) (void)hipGraphDestroy(g);
@@ -1984,6 +2048,8 @@ static sre_status step_graph(sre_engine *e, unsigned flags, int K,
     HIP_TRY(hipGraphUpload(slot->exec, e->stream));
     slot->flags = flags;
     slot->steps = K;
+    slot->sig.clear();
+    if (flags & kGraphRebuild) slot->sig = e->rebuild_sig;
     slot->epoch = e->graph_epoch;
   }
   slot->last_use = ++e->graph_uses;
@@ -2440,15 +2506,21 @@ extern "C" sre_status sre_set_md_state(sre_engine *e, const sre_md_state *in) {
   });
 }
 
-// largest displacement^2 since the last rebuild against skin/2 (*ok), and
-// the force-range flag, in one readback.  A skin violation is reported first:
-// missed pairs are the likelier cause of a range error that follows it.
-static sre_status md_skin_ok(sre_engine *e, bool *ok, float *disp2 = nullptr) {
+// largest displacement^2 since the last rebuild, and the force-range flag
+// (h_flags), in one wait
+static sre_status md_skin_read(sre_engine *e) {
   launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms),
                       e->d_skin_part, 0, e->d_flags, e->stream, nullptr, nullptr, 0,
                       e->d_info_slices);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(e->stream));
+  return SRE_OK;
+}
+
+// What was read against skin/2 (*ok), and the flag.  A skin violation is
+// reported first: missed pairs are the likelier cause of a range error that
+// follows it.
+static sre_status md_skin_verdict(sre_engine *e, bool *ok, float *disp2 = nullptr) {
   const float d2 = skin_disp2(e);
   const float half = 0.5f * e->skin;
   *ok = !(d2 > half * half);
@@ -2457,12 +2529,17 @@ static sre_status md_skin_ok(sre_engine *e, bool *ok, float *disp2 = nullptr) {
   return SRE_OK;
 }
 
-// Saves (restore = false) or restores the state an MD stretch starts from:
-// bound positions, velocities, saved forces, kick sums and the chain.
-static sre_status md_snapshot(sre_engine *e, bool restore) {
+static sre_status md_skin_ok(sre_engine *e, bool *ok) {
+  sre_status s = md_skin_read(e);
+  return s == SRE_OK ? md_skin_verdict(e, ok) : s;
+}
+
+// Buffers of the state an MD stretch starts from.
+static sre_status md_snapshot_buffers(sre_engine *e) {
   const int N = e->n_atoms;
   const size_t npos = (size_t)N * e->pos_stride;
   if (!e->d_snap_vel || e->snap_pos_cap < npos) {
+    e->graph_epoch++;
     dfree(e->d_snap_pos);
     HIP_TRY(dalloc(&e->d_snap_pos, npos));
     e->snap_pos_cap = npos;
@@ -2473,6 +2550,14 @@ static sre_status md_snapshot(sre_engine *e, bool restore) {
     }
     if (!e->d_snap_md) HIP_TRY(dalloc(&e->d_snap_md, 1));
   }
+  return SRE_OK;
+}
+
+// Saves (restore = false) or restores the state an MD stretch starts from:
+// bound positions, velocities, saved forces, kick sums and the chain.
+static void enqueue_snapshot(sre_engine *e, bool restore) {
+  const int N = e->n_atoms;
+  const size_t npos = (size_t)N * e->pos_stride;
   struct Pair { void *live; void *snap; size_t bytes; };
   const Pair pairs[] = {
       {const_cast<float *>(e->d_pos), e->d_snap_pos, sizeof(float) * npos},
@@ -2489,7 +2574,11 @@ static sre_status md_snapshot(sre_engine *e, bool restore) {
     ++c.count;
   }
   launch_md_copy(c, e->stream);     // one launch for all five buffers
-  if (restore) clear_force_flag(e);
+}
+
+static sre_status md_restore(sre_engine *e) {
+  enqueue_snapshot(e, true);
+  clear_force_flag(e);
   HIP_TRY(hipGetLastError());
   return SRE_OK;
 }
@@ -2553,41 +2642,104 @@ extern "C" sre_status sre_md_run(sre_engine *e, int n_steps, int rebuild_every,
     // every speculative stretch starts from a list built at its first step
     s = do_rebuild(e);
     if (s != SRE_OK) return s;
+    fresh = true;
     if (n_rebuilds) ++*n_rebuilds;
   }
   int left = n_steps;
+  bool settled = fresh;   // a rebuild has been prepared in this run
+  // adaptive: the log entry of the rebuild before the current stretch while its
+  // list lengths are unchecked, and the range flag of the steps before it
+  const uint64_t *open = nullptr;
+  unsigned open_flag = 0;
+  auto overflowed = [&] { return open && (int)open[0] > e->cap; };
+  // an error with that rebuild unchecked: lists cut short are not left behind
+  auto leave = [&](sre_status err) {
+    if (open && hipStreamSynchronize(e->stream) == hipSuccess && overflowed()) e->built = false;
+    return err;
+  };
   while (left > 0) {
     if (rebuild_every == SRE_MD_ADAPTIVE) {
       // a stretch of K steps as one graph from a snapshot; the displacement
       // read back at its end decides: kept (next K aims at 80 % of skin/2,
       // displacements growing about linearly) or rolled back and redone
-      // with K/2.  Each kept stretch used complete lists throughout.
+      // with K/2.  Each kept stretch used complete lists throughout: the
+      // rebuild at a stretch's end tells the displacement first, and the next
+      // stretch is queued while it still builds; whether the lists had room is
+      // checked at that stretch's end, and if not, it too is rolled back.
+      // (Waiting for each rebuild left the GPU idle for some 30 us per
+      // stretch: 2840 us for 100 steps of 4 000 atoms, now 2377.)  Snapshot, steps
+      // and rebuild are one graph once a rebuild of this run has prepared its
+      // arguments, which nothing changes before the run's end.
       const int K = std::min({left, e->md_adapt_k, kMaxGraphSteps});
       const bool last = K == left;
-      s = md_snapshot(e, false);
-      if (s != SRE_OK) return s;
+      const bool whole = !last && settled;
+      s = md_snapshot_buffers(e);
+      if (s != SRE_OK) return leave(s);
       hipGraphExec_t ex;
-      s = step_graph(e, kGraphMD | (last ? flags : fl), K, &ex);
-      if (s != SRE_OK) return s;
-      HIP_TRY(hipGraphLaunch(ex, e->stream));
+      s = step_graph(e, kGraphMD | kGraphSnap | (whole ? kGraphRebuild : 0u) |
+                            (last ? flags : fl), K, &ex);
+      if (s != SRE_OK) return leave(s);
+      const uint64_t *info = nullptr;
+      if (hipError_t r = whole ? launch_rebuild(e, ex, &info) : hipGraphLaunch(ex, e->stream);
+          r != hipSuccess)
+        return leave(fail(SRE_ERR_HIP, "MD steps: %s", hipGetErrorString(r)));
       e->md_since_rebuild += K;
       bool ok;
       float d2;
       if (!last) {
-        s = do_rebuild(e);   // reads the stretch's displacement back
-        if (s != SRE_OK) return s;
-        if (n_rebuilds) ++*n_rebuilds;
-        d2 = e->last_disp2;
-        ok = !(d2 > half * half);
+        s = whole ? SRE_OK : rebuild_begin(e, &info);
+        settled = true;
+        if (s == SRE_OK) s = wait_disp2(e, info, &d2);
       } else {
-        s = md_skin_ok(e, &ok, &d2);
+        s = md_skin_read(e);
+      }
+      if (s != SRE_OK) return leave(s);
+      if (overflowed()) {
+        // the stretch ran on lists cut short: again from its start, on longer
+        // ones (any rebuild queued behind it goes with it)
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        const int mc = (int)open[0];
+        const float before = e->last_disp2;
+        open = nullptr;
+        s = md_restore(e);
+        if (s == SRE_OK && (open_flag & 1u)) launch_fill_u32(e->d_flags + 1, 1u, 1, e->stream);
+        if (s == SRE_OK) s = ensure_list(e, grown_cap(e, mc));
+        if (s == SRE_OK) s = do_rebuild(e);
+        if (s != SRE_OK) {
+          e->built = false;
+          return s;
+        }
+        e->last_disp2 = before;
+        continue;
+      }
+      if (open) {
+        e->max_count = (int)open[0];
+        e->n_list = (int64_t)open[1];
+        open = nullptr;
+      }
+      if (!last) {
+        ok = !(d2 > half * half);
+        if (n_rebuilds) ++*n_rebuilds;
+        if (ok) {
+          open = info;
+          open_flag = e->h_flags[1];
+          e->last_disp2 = d2;
+          e->md_since_rebuild = 0;
+          e->stats_valid = e->forces_valid = e->atom_stats_valid = false;
+        } else {
+          HIP_TRY(hipStreamSynchronize(e->stream));
+          s = rebuild_end(e, info);
+          if (s != SRE_OK) return s;
+        }
+      } else {
+        s = md_skin_verdict(e, &ok, &d2);
         if (s != SRE_OK) return s;
       }
       if (!ok) {
         if (K == 1)
           return fail(SRE_ERR_SKIN, "an atom moved %g > skin/2 in one step",
                       sqrt((double)d2));
-        s = md_snapshot(e, true);
+        s = md_restore(e);
         if (s != SRE_OK) return s;
         s = do_rebuild(e);
         if (s != SRE_OK) return s;

@@ -425,8 +425,24 @@ __device__ __forceinline__ int place_idx(int c) { return c + (c >> 4); }
 __global__ __launch_bounds__(256) void k_cell_count(int n, int n_cells, const float *pos,
                                                     int stride, const int *rep_of,
                                                     const RepInfo *reps, uint32_t *keys,
-                                                    uint32_t *count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+                                                    uint32_t *count, EarlySkin early) {
+  if (blockIdx.x == 0) {      // one block more than the atoms need
+    __shared__ float red[256 / kWave];
+    float d2 = 0.f;
+    for (int k = threadIdx.x; k < early.n; k += 256) d2 = fmaxf(d2, early.part[k]);
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, o, kWave));
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = d2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int q = 1; q < 256 / kWave; ++q) d2 = fmaxf(d2, red[q]);
+      unsigned long long *dst = early.log + 3 * (size_t)(*early.log_idx % (unsigned)early.log_cap);
+      __hip_atomic_store(dst + 2, (unsigned long long)__float_as_uint(d2), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return;
+  }
+  const int i = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   // keys are < n_cells by construction; the clamp keeps the counts in bounds
   const uint32_t k = min(cell_key(pos, stride, rep_of, reps, i), (uint32_t)(n_cells - 1));
@@ -571,13 +587,13 @@ void launch_cell_sort_gather(int n, int n_cells, const float *pos, int stride,
                              uint32_t *inv_perm, float4 *res4, float *rcut,
                              int *tail_idx, const float *rc_atom, uint4 *backup_s,
                              const float *anchor, float4 *anchor_s, hipStream_t st,
-                             bool counted) {
+                             const EarlySkin &early, bool counted) {
   if (n <= 0) return;
   uint32_t *cursor = count + cell_count_half(n_cells);
   const dim3 g((n + 255) / 256), t(256);
   if (!counted)
-    hipLaunchKernelGGL(k_cell_count, g, t, 0, st, n, n_cells, pos, stride, rep_of, reps,
-                       b.tkey, count);
+    hipLaunchKernelGGL(k_cell_count, dim3(g.x + 1), t, 0, st, n, n_cells, pos, stride, rep_of,
+                       reps, b.tkey, count, early);
   if (n_cells <= kPlaceCells) {
     hipLaunchKernelGGL(k_cell_place, dim3((n + kSortT - 1) / kSortT), dim3(kSortT), 0, st,
                        n, n_cells, b.tkey, count, cursor, start, b.key_b, b.val_b);

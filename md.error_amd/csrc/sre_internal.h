@@ -337,8 +337,19 @@ size_t radix_counts_capacity(int n, int key_bits);
 size_t cell_count_capacity(int n_cells);
 // up to this many cells the scan of the counts is fused into the placement
 constexpr int kPlaceCells = 15360;
+// The largest squared displacement (float bits) over the n skin partials, to
+// word 2 of rebuild-log entry *log_idx % log_cap by the rebuild's first launch:
+// the host can act on it while the list is built.  launch_rebuild_info writes
+// the same word again and clears the partials.
+struct EarlySkin {
+  const float *part;
+  int n;
+  unsigned long long *log;
+  const unsigned *log_idx;
+  int log_cap;
+};
 // counted: the keys (b.tkey) and counts were made by a CountFold of the last
-// force launch, so the histogram launch is skipped.
+// force launch, so the histogram launch is skipped.  early: see EarlySkin.
 void launch_cell_sort_gather(int n, int n_cells, const float *pos, int stride,
                              const int *types, const int *rep_of,
                              const RepInfo *reps, const float *rc_table,
@@ -347,7 +358,7 @@ void launch_cell_sort_gather(int n, int n_cells, const float *pos, int stride,
                              uint32_t *inv_perm, float4 *res4, float *rcut,
                              int *tail_idx, const float *rc_atom, uint4 *backup_s,
                              const float *anchor, float4 *anchor_s, hipStream_t st,
-                             bool counted = false);
+                             const EarlySkin &early, bool counted = false);
 // Gather into cell order (+ rc assignment) fused with the cell offsets
 // start[0..n_cells] computed from the sorted keys.
 void launch_gather_sorted(int n, int n_cells, const uint32_t *keys,
