@@ -364,10 +364,14 @@ __device__ __forceinline__ int wave_max_int(int v) {
 // (acc_floor, sre_internal.h); the lane value is bits(acc) - bits(C).
 //
 // One wave-tile (64/T consecutive sorted atoms) of the force evaluation;
-// `wave` is the tile index.
-template <int T, int U, bool STATS, bool TAIL, bool MULTI, bool SHIFT>
+// `wave` is the tile index.  W > 1: the block's W wavefronts share the tile,
+// wavefront `part` taking the part-th of W runs of its groups; the forces of
+// the parts are added in LDS (exact integers, so the split does not change
+// them) and the first wavefront stores them.
+template <int T, int U, bool STATS, bool TAIL, bool MULTI, bool SHIFT, int W = 1>
 __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *sp,
-                                           const int wave) {
+                                           const int wave, const int part = 0) {
+  static_assert(W == 1 || !STATS, "the FP32 sums depend on the split");
   constexpr int A = kWave / T;
   const int lane = threadIdx.x & (kWave - 1);
   const int l = lane % T;
@@ -465,13 +469,15 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *
   // there: it is clamped to a valid atom and its pair is masked in
   // eval_group.
   const unsigned nmax = (unsigned)(a.n - 1);
+  const int per = W > 1 ? (groups + W - 1) / W : groups;
+  const int g0 = W > 1 ? part * per : 0, g1 = W > 1 ? min(groups, g0 + per) : groups;
   auto prefetch = [&](uint4 *p, int *jr, int g) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
       p[u] = gather_pos_idx<MULTI>(prs, (int)min((unsigned)jr[u], nmax));
     // (rows of groups past the wave's last one: its last rows again, cache
     // hits, so no row past the wave's lists is fetched)
-    const int gr = max(min(g + 2, groups - 1), 0);
+    const int gr = max(min(g + 2, g1 - 1), g0);
 #pragma unroll
     for (int u = 0; u < U; ++u) jr[u] = row(gr * U + u);
     asm volatile("" ::: "memory");
@@ -479,28 +485,28 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *
   int ja[U], jb[U];   // list rows of the groups due in buffers a and b
   uint4 pa[U], pb[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) ja[u] = row(u);
+  for (int u = 0; u < U; ++u) ja[u] = row(g0 * U + u);
 #pragma unroll
-  for (int u = 0; u < U; ++u) jb[u] = row(U + u);
+  for (int u = 0; u < U; ++u) jb[u] = row((g0 + 1) * U + u);
   // issue order at the loop entry as on the back edge (rows of g+1, then
   // the gathers of g and the rows of g+2), so that the loop waits only for
   // the loads it is about to use
   asm volatile("" ::: "memory");
-  prefetch(pa, ja, 0);
+  prefetch(pa, ja, g0);
   // the accumulators' FP64 adds round toward zero inside the pair loop
   // (FP32 rounding is a separate field of the mode register, untouched)
   round_f64_toward_zero();
   // whole pairs of groups in the loop (no branch inside its body, so the
   // loads of each half are waited for only where they are used), the odd
   // last group after it
-  int g = 0;
-  for (; g + 1 < groups; g += 2) {
+  int g = g0;
+  for (; g + 1 < g1; g += 2) {
     prefetch(pb, jb, g + 1);
     eval_group(pa, g);
     prefetch(pa, ja, g + 2);
     eval_group(pb, g + 1);
   }
-  if (g < groups) eval_group(pa, g);  // wave-uniform
+  if (g < g1) eval_group(pa, g);  // wave-uniform
   round_f64_nearest();
   const int64_t acc0 = __double_as_longlong(kAccBase);
   int64_t Fx = __double_as_longlong(ax) - acc0;
@@ -509,6 +515,27 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *
   Fx = group_sum(Fx, T);
   Fy = group_sum(Fy, T);
   Fz = group_sum(Fz, T);
+  if (W > 1) {
+    __shared__ int64_t s_f[W > 1 ? W - 1 : 1][3][A];
+    __shared__ float s_abs[W > 1 ? W - 1 : 1][kWave];
+    if (part > 0) {
+      if (l == 0) {
+        s_f[part - 1][0][lane / T] = Fx;
+        s_f[part - 1][1][lane / T] = Fy;
+        s_f[part - 1][2][lane / T] = Fz;
+      }
+      s_abs[part - 1][lane] = fsabs;
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int w = 0; w < W - 1; ++w) {
+      Fx += s_f[w][0][lane / T];
+      Fy += s_f[w][1][lane / T];
+      Fz += s_f[w][2][lane / T];
+      fsabs += s_abs[w][lane];     // the unsplit lane's sum, for the same check
+    }
+  }
   // every lane's sum of |pair component| * 2^32 is at most rc * sum |fs|
   // (each component is fs * d with |d| < rc), and must stay below 2^51 for
   // the accumulators to stay in [2^52, 2^53); 2^50 leaves room for the FP32
@@ -576,6 +603,28 @@ __global__ __launch_bounds__(256) void k_force_mixed(ForceArgs a) {
   const int per = (n_tiles + a.persist_waves - 1) / a.persist_waves;
   const int t0 = wave * per, t1 = min(n_tiles, t0 + per);
   for (int t = t0; t < t1; ++t) force_tile<T, U, STATS, TAIL, MULTI, SHIFT>(a, sp, t);
+}
+
+// One tile per block of kRowWaves wavefronts (see force_tile): with at most one
+// tile per SIMD a wavefront of its own leaves each SIMD waiting for one chain
+// of gathers.  Tile per wavefront / per block of 4: 4.4 / 3.8 us at 1 000 atoms,
+// 4.6 / 4.2 at 4 000, 5.6 / 4.4 on an 8 000-atom slab, 5.6 / 5.2 at 16 000, 40.7
+// / 37.3 at 16 000 atoms with 1 366 list entries each; with two tiles per SIMD
+// 6.7 / 6.3 but 71.0 / 72.8 on such long lists, with four 8.9 / 9.9.  (2 and 8
+// wavefronts lie between or behind.)
+constexpr int kRowWaves = 4;
+template <int T, bool TAIL, bool MULTI>
+__global__ __launch_bounds__(kWave * kRowWaves) void k_force_mixed_rows(ForceArgs a) {
+  if (a.ctr_out && blockIdx.x == 0 && threadIdx.x == 0) *a.ctr_out = *a.ctr_in + 1;
+  __shared__ PairParam sp[MULTI ? kMaxPairTypes : 1];
+  if (MULTI) {
+    for (int t = threadIdx.x; t < a.n_types * a.n_types; t += blockDim.x)
+      sp[t] = a.params[t];
+    __syncthreads();
+  }
+  const int tile = a.xcd_remap ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+  force_tile<T, 2, false, TAIL, MULTI, false, kRowWaves>(
+      a, sp, tile, __builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
 }
 
 // ------------------------------------------------- cell-window form ----
@@ -995,12 +1044,25 @@ static void launch_mixed_u(int grid, int block, bool multi, const ForceArgs &a,
     launch_mixed_s<T, U, STATS, TAIL, false>(grid, block, multi, a, st);
 }
 
+
 template <int T, bool STATS, bool TAIL>
 static void launch_force_t(int precision, int unroll, int block,
                            const ForceArgs &a, hipStream_t st) {
   const int waves = force_num_waves(a.n, T);
-  int grid = (waves * kWave + block - 1) / block;
   const bool multi = a.n_types > 1;
+  // at most one tile per SIMD (both sides at k_force_mixed_rows); the
+  // statistics' FP32 sums would depend on the split, and the launches with
+  // blocks in front, or persistent, have enough wavefronts
+  if constexpr (!STATS) {
+    if (precision == 0 && waves <= a.n_simd && a.persist_waves <= 0 && !a.next.active &&
+        a.count.n_blocks == 0) {
+      const dim3 grid(waves), threads(kWave * kRowWaves);
+      if (multi) hipLaunchKernelGGL((k_force_mixed_rows<T, TAIL, true>), grid, threads, 0, st, a);
+      else hipLaunchKernelGGL((k_force_mixed_rows<T, TAIL, false>), grid, threads, 0, st, a);
+      return;
+    }
+  }
+  int grid = (waves * kWave + block - 1) / block;
   if (precision == 0 && a.persist_waves > 0) grid = a.persist_waves * kWave / block;
   // the next step's refresh and the next rebuild's histogram: blocks of their
   // own in front (multiples of 8, so each force block keeps its XCD)

@@ -580,6 +580,7 @@ struct ForceArgs {
   double *fxd, *fyd, *fzd;     // FP64 output (sorted order)
   double *atom_stats;          // optional per-atom (E, Wxx, Wyy, Wzz)
   unsigned *err_flag;
+  int n_simd;          // of the device (0: no launch that depends on it)
   // perturbation step counter: one thread writes *ctr_out = *ctr_in + 1
   // (ctr_in == ctr_out, or two slots when the launch refreshes the next
   // step from *ctr_in); NULL = none
