@@ -242,7 +242,7 @@ typedef struct {
                            persistent launch of k wavefronts per SIMD, each taking a
                            contiguous chunk of tiles (same sums) */
   int sort_mode;        /* binning at a rebuild (same cell order in every mode):
-                           0 = counting sort by cell up to 15360 cells, radix sort
+                           0 = counting sort by cell up to 30720 cells, radix sort
                            above; 1 = LSD radix sort of the cell key; 2 = counting
                            sort at any cell count */
   int force_mode;       /* mixed form: 0 = neighbor-list kernel; 1 = cell-window

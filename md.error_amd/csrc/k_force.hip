@@ -147,7 +147,7 @@ __device__ __forceinline__ bool force_block(const ForceArgs &a, int *bid, int *n
                                         a.reps, i),
                                (uint32_t)(a.count.n_cells - 1));
         a.count.keys[i] = k;
-        atomicAdd(&a.count.count[k], 1u);
+        a.count.place[i] = atomicAdd(&a.count.count[k], 1u);
       }
       return false;
     }

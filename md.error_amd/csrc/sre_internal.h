@@ -331,12 +331,12 @@ size_t radix_counts_capacity(int n, int key_bits);
 // Counting sort by cell and gather into cell order (+ rc assignment): the
 // same permutation (val_a), cell offsets start[0..n_cells] and gathered data
 // as the radix sort followed by launch_gather_sorted.  count (the cell
-// counts and the placement cursors) holds cell_count_capacity(n_cells) zeros
-// before the call and again after it; uses b.tkey, b.key_b, b.val_b as
-// scratch.
+// counts) holds cell_count_capacity(n_cells) zeros before the call and again
+// after it; uses b.tkey, b.tval, b.key_b, b.val_b as scratch.
 size_t cell_count_capacity(int n_cells);
 // up to this many cells the scan of the counts is fused into the placement
 constexpr int kPlaceCells = 15360;
+constexpr int kCountCells = 30720;   // the counting sort's, by default
 // The largest squared displacement (float bits) over the n skin partials, to
 // word 2 of rebuild-log entry *log_idx % log_cap by the rebuild's first launch:
 // the host can act on it while the list is built.  launch_rebuild_info writes
@@ -348,7 +348,7 @@ struct EarlySkin {
   const unsigned *log_idx;
   int log_cap;
 };
-// counted: the keys (b.tkey) and counts were made by a CountFold of the last
+// counted: the keys (b.tkey), places (b.tval) and counts were made by a CountFold of the last
 // force launch, so the histogram launch is skipped.  early: see EarlySkin.
 void launch_cell_sort_gather(int n, int n_cells, const float *pos, int stride,
                              const int *types, const int *rep_of,
@@ -550,14 +550,14 @@ struct NextRefresh {
 // force launch, done by blocks in front of that launch when it is the last
 // of a segment (it does not move the atoms, so the keys are those the
 // rebuild would compute): one atom per thread, caller order, keys[i] and
-// count[key] += 1 as k_cell_count.
+// place[i] = count[key]++ as k_cell_count.
 struct CountFold {
   int n_blocks;                // 0 = none; else a multiple of 8
   const float *pos;            // caller positions
   int stride;
   const int *rep_of;
   int n_cells;
-  uint32_t *keys, *count;
+  uint32_t *keys, *place, *count;
 };
 
 struct ForceArgs {
