@@ -994,19 +994,21 @@ static void enqueue_rebuild(sre_engine *e, int n_parts, hipStream_t st,
   const int N = e->n_atoms;
   const float *anchor = e->pert_anchored ? e->d_anchor : nullptr;
   const float *rc_atom = e->rc_explicit ? e->d_rc_atom : nullptr;
+  const int *rep_of = e->n_rep > 1 ? e->d_rep_of : nullptr;
+  const int *types = e->n_types > 1 ? e->d_types : nullptr;
   if (counting_sort(e)) {
-    launch_cell_sort_gather(N, e->n_cells, e->d_pos, e->pos_stride, e->d_types,
-                            e->d_rep_of, e->d_reps, e->d_rc, e->n_types, e->sb,
+    launch_cell_sort_gather(N, e->n_cells, e->d_pos, e->pos_stride, types,
+                            rep_of, e->d_reps, e->d_rc, e->n_types, e->sb,
                             e->d_cell_count, e->d_start, e->d_pos4, e->d_backup,
                             e->d_inv_perm, e->d_res4, e->d_rcut, e->d_tail_idx,
                             rc_atom, e->d_backup_s, anchor, e->d_anchor_s, st,
                             EarlySkin{e->d_skin_part, skin_part_count(N), e->d_log,
                                       e->d_log_idx, kRebuildLog}, counted);
   } else {
-    launch_radix_sort(N, e->key_bits, e->d_pos, e->pos_stride, e->d_rep_of,
+    launch_radix_sort(N, e->key_bits, e->d_pos, e->pos_stride, rep_of,
                       e->d_reps, e->sb, st);
     launch_gather_sorted(N, e->n_cells, e->sb.key_a, e->sb.val_a, e->d_pos,
-                         e->pos_stride, e->d_types, e->d_rep_of, e->d_reps,
+                         e->pos_stride, types, rep_of, e->d_reps,
                          e->d_rc, e->n_types, e->d_start, e->d_pos4, e->d_backup,
                          e->d_inv_perm, e->d_res4, e->d_rcut, e->d_tail_idx,
                          rc_atom, st, e->d_backup_s, anchor, e->d_anchor_s);
@@ -1961,7 +1963,7 @@ static sre_status enqueue_fused_steps(sre_engine *e, unsigned flags, int K,
       a.count.n_blocks = nx.n_blocks;
       a.count.pos = e->d_pos;
       a.count.stride = e->pos_stride;
-      a.count.rep_of = e->d_rep_of;
+      a.count.rep_of = e->n_rep > 1 ? e->d_rep_of : nullptr;
       a.count.n_cells = e->n_cells;
       a.count.keys = e->sb.tkey;
       a.count.place = e->sb.tval;

@@ -131,11 +131,12 @@ __host__ __device__ inline int cell_of(uint32_t u, int nc) {
 }
 
 // Cell key of atom i: replica cell offset + (cx, cy, cz) with z fastest, so a
-// column of cells is one contiguous range of sorted atoms.
+// column of cells is one contiguous range of sorted atoms.  rep_of: NULL with
+// one replica.
 __device__ __forceinline__ uint32_t cell_key(const float *pos, int stride,
                                              const int *rep_of,
                                              const RepInfo *reps, int i) {
-  const RepInfo &R = reps[rep_of[i]];
+  const RepInfo &R = reps[rep_of ? rep_of[i] : 0];
   const float *p = pos + (size_t)i * stride;
   const int cx = cell_of(quantize(p[0], R.invq[0]), R.nc[0]);
   const int cy = cell_of(quantize(p[1], R.invq[1]), R.nc[1]);
@@ -360,7 +361,8 @@ void launch_cell_sort_gather(int n, int n_cells, const float *pos, int stride,
                              const float *anchor, float4 *anchor_s, hipStream_t st,
                              const EarlySkin &early, bool counted = false);
 // Gather into cell order (+ rc assignment) fused with the cell offsets
-// start[0..n_cells] computed from the sorted keys.
+// start[0..n_cells] computed from the sorted keys.  In both gathers types may
+// be NULL with one type, rep_of with one replica.
 void launch_gather_sorted(int n, int n_cells, const uint32_t *keys,
                           const uint32_t *perm, const float *pos, int stride,
                           const int *types, const int *rep_of,
