@@ -460,7 +460,7 @@ void launch_tail_weights(int n, int n_entries, const int *tail_idx, const uint32
 // Geometric integrals of one species profile: F = sum over bins/images of
 // rho*(G(s1)-G(s0)) split into the sigma^6 and sigma^12 parts, likewise the
 // energy integral of P, and their derivatives with respect to R.
-constexpr int kTailAdjBlock = 128;  // threads per tail bin in the adjoint
+constexpr int kTailAdjBlock = 256;  // threads per tail bin in the adjoint
 
 struct TailX {
   double F6, F12, E6, E12, dF6, dF12, dE6, dE12;
@@ -568,15 +568,22 @@ __device__ TailX tail_x_finish(double z, double R, int nz, double Lz,
 }
 
 // One block per tail bin (over all replicas), its threads splitting the
-// planar integrals (fixed-order tree reduction): combines the per-entry
+// planar integrals (fixed-order reduction): combines the per-entry
 // weights W_F = sum g_z and W_E = sum dLdE with the derivatives of the table
 // entries.  Writes d/drc of the bin to g_rc and the eps/sigma parts to
-// contrib[bin][2*npt].
+// contrib[bin][2*npt].  What bounds it: FP64 divisions, in a chain of six
+// integrands per thread, and the one-thread ends.  The integrals depend on the
+// bin and the other atom's species alone: one pass for each of those, their
+// remainders by one thread each at once, then one thread per pair type (a pass
+// per pair type, each with its own tree of barriers and one-thread end, took
+// 33 us for 256 bins of two species, now 16).
 __global__ __launch_bounds__(kTailAdjBlock) void k_adjoint_tail(
     int n_bins, const int *entry_rep, const RepInfo *reps, int n_types,
     const PairParamD *params, const float *rc_table, const double *rho,
     const int64_t *wts, double *contrib, double *g_rc) {
-  __shared__ double red[9][kTailAdjBlock];
+  __shared__ double red[kMaxTypes][kTailAdjBlock / kWave][9];
+  __shared__ TailX sx[kMaxTypes];
+  __shared__ double sg_rc[kMaxPairTypes];
   const int bg = blockIdx.x;
   const int t = threadIdx.x;
   const int npt = n_types * n_types;
@@ -588,46 +595,57 @@ __global__ __launch_bounds__(kTailAdjBlock) void k_adjoint_tail(
   const double z = (bin + 0.5) * Lz / nz;
   const double rc = (double)rc_table[R.rc_off + bin];
   double *c = contrib + (size_t)bg * 2 * npt;
-  if (t == 0)
-    for (int k = 0; k < 2 * npt; ++k) c[k] = 0.0;
-  double grc = 0.0;
-  for (int ta = 0; ta < n_types; ++ta) {
+  for (int tb = 0; tb < n_types; ++tb) {
+    double acc[9];
+    tail_x_part(z, rc, rho + R.rho_off + (size_t)tb * R.rho_nz, R.rho_nz, Lz,
+                t, kTailAdjBlock, acc);
+    for (int k = 0; k < 9; ++k) {
+#pragma unroll
+      for (int o = kWave / 2; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o, kWave);
+      if (t % kWave == 0) red[tb][t / kWave][k] = acc[k];
+    }
+  }
+  __syncthreads();
+  if (t < n_types) {
+    double acc[9];
+    for (int k = 0; k < 9; ++k) {
+      acc[k] = red[t][0][k];
+      for (int q = 1; q < kTailAdjBlock / kWave; ++q) acc[k] += red[t][q][k];
+    }
+    sx[t] = tail_x_finish(z, rc, R.rho_nz, Lz, acc);
+  }
+  __syncthreads();
+  for (int p = t; p < npt; p += kTailAdjBlock) {
+    const int ta = p / n_types, tb = p % n_types;
     const int te = bg * n_types + ta;
     const double WF = (double)wts[2 * (size_t)te] * kFixInv;
     const double WE = (double)wts[2 * (size_t)te + 1] * kFixInv;
-    if (WF == 0.0 && WE == 0.0) continue;  // block-uniform
-    for (int tb = 0; tb < n_types; ++tb) {
-      double acc[9];
-      tail_x_part(z, rc, rho + R.rho_off + (size_t)tb * R.rho_nz, R.rho_nz, Lz,
-                  t, kTailAdjBlock, acc);
-      for (int k = 0; k < 9; ++k) red[k][t] = acc[k];
-      __syncthreads();
-      for (int o = kTailAdjBlock / 2; o > 0; o >>= 1) {
-        if (t < o)
-          for (int k = 0; k < 9; ++k) red[k][t] += red[k][t + o];
-        __syncthreads();
-      }
-      if (t == 0) {
-        for (int k = 0; k < 9; ++k) acc[k] = red[k][0];
-        const TailX x = tail_x_finish(z, rc, R.rho_nz, Lz, acc);
-        const PairParamD &P = params[ta * n_types + tb];
-        const double sg = P.sig, ep = P.eps;
-        const double s2 = sg * sg, s6 = s2 * s2 * s2, s12 = s6 * s6;
-        // T_F = -2 pi eps (s6 F6 + s12 F12),  T_E = eps/2 (s6 E6 + s12 E12)
-        const double cF = -6.283185307179586, cE = 0.5;
-        const double tF = s6 * x.F6 + s12 * x.F12, tE = s6 * x.E6 + s12 * x.E12;
-        const double ds6 = 6.0 * s6 / sg, ds12 = 12.0 * s12 / sg;
-        const int p = ta * n_types + tb;
-        c[p] += WF * cF * tF + WE * cE * tE;
-        c[npt + p] += ep * (WF * cF * (ds6 * x.F6 + ds12 * x.F12) +
-                            WE * cE * (ds6 * x.E6 + ds12 * x.E12));
-        grc += ep * (WF * cF * (s6 * x.dF6 + s12 * x.dF12) +
-                     WE * cE * (s6 * x.dE6 + s12 * x.dE12));
-      }
-      __syncthreads();  // red[] reused
+    double ceps = 0.0, csig = 0.0, grc = 0.0;
+    if (WF != 0.0 || WE != 0.0) {
+      const TailX x = sx[tb];
+      const PairParamD &P = params[p];
+      const double sg = P.sig, ep = P.eps;
+      const double s2 = sg * sg, s6 = s2 * s2 * s2, s12 = s6 * s6;
+      // T_F = -2 pi eps (s6 F6 + s12 F12),  T_E = eps/2 (s6 E6 + s12 E12)
+      const double cF = -6.283185307179586, cE = 0.5;
+      const double tF = s6 * x.F6 + s12 * x.F12, tE = s6 * x.E6 + s12 * x.E12;
+      const double ds6 = 6.0 * s6 / sg, ds12 = 12.0 * s12 / sg;
+      ceps = WF * cF * tF + WE * cE * tE;
+      csig = ep * (WF * cF * (ds6 * x.F6 + ds12 * x.F12) +
+                   WE * cE * (ds6 * x.E6 + ds12 * x.E12));
+      grc = ep * (WF * cF * (s6 * x.dF6 + s12 * x.dF12) +
+                  WE * cE * (s6 * x.dE6 + s12 * x.dE12));
     }
+    c[p] = ceps;
+    c[npt + p] = csig;
+    sg_rc[p] = grc;
   }
-  if (t == 0) g_rc[R.rc_off + bin] = grc;
+  __syncthreads();
+  if (t == 0) {
+    double grc = 0.0;
+    for (int p = 0; p < npt; ++p) grc += sg_rc[p];
+    g_rc[R.rc_off + bin] = grc;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_adjoint_tail_reduce(
