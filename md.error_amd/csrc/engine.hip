@@ -171,6 +171,7 @@ struct sre_engine {
   // write, so that a check is one wait and no copy
   volatile unsigned *h_flags = nullptr;
   unsigned *d_flags = nullptr;  // its device address
+  unsigned *d_skin_ticket = nullptr;   // blocks of a refresh that are done
   uint64_t *d_step_ctr = nullptr;  // perturbation step counter (graph mode)
   float pert_sigma = 0.f;
   uint64_t pert_seed = 0;
@@ -271,7 +272,7 @@ sre_engine::~sre_engine() {
   if (h_log) (void)hipHostFree(h_log);
   dfree(d_log_idx);
   dfree(d_fyd); dfree(d_fzd); dfree(d_nin); dfree(d_stat_part); dfree(d_stat_ticket);
-  dfree(d_atom_stats); dfree(d_tmp_out); dfree(d_step_ctr);
+  dfree(d_atom_stats); dfree(d_tmp_out); dfree(d_step_ctr); dfree(d_skin_ticket);
   dfree(d_anchor); dfree(d_skin_part); dfree(d_build_part); dfree(d_info_slices);
   dfree(d_pos4_alt); dfree(d_res4_alt); dfree(d_backup_s); dfree(d_anchor_s);
   dfree(d_adj); dfree(d_adj_tw);
@@ -346,6 +347,8 @@ extern "C" sre_status sre_create(sre_engine **out, const sre_options *opt) {
     memset(flags, 0, 4 * sizeof(unsigned));
     r = hipHostGetDevicePointer((void **)&e->d_flags, flags, 0);
   }
+  if (r == hipSuccess) r = dalloc(&e->d_skin_ticket, 1);
+  if (r == hipSuccess) r = hipMemsetAsync(e->d_skin_ticket, 0, sizeof(unsigned), e->stream);
   if (r == hipSuccess) r = dalloc(&e->d_counters, 3);
   if (r == hipSuccess) r = hipMemsetAsync(e->d_counters, 0, 3 * sizeof(uint64_t), e->stream);
   if (r == hipSuccess) r = hipHostMalloc((void **)&e->h_info, 4 * sizeof(uint64_t), hipHostMallocDefault);
@@ -1184,20 +1187,27 @@ static float skin_disp2(const sre_engine *e) {
   return d2;
 }
 
+// Queues the refresh of the lattice copy from the bound positions; skin: and
+// the largest displacement^2 into h_flags.
+static void enqueue_refresh(sre_engine *e, bool skin) {
+  const bool fold = skin && e->n_atoms <= kSkinFoldAtoms;
+  launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
+                          e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
+                          e->d_res4, e->d_skin_part, nullptr, e->stream,
+                          fold ? SkinNow{e->d_skin_ticket, e->d_flags} : SkinNow{});
+  if (skin && !fold)
+    launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms), e->d_skin_part, 0,
+                        e->d_flags, e->stream, nullptr, nullptr, 0, e->d_info_slices);
+}
+
 extern "C" sre_status sre_update_positions(sre_engine *e, int *need_rebuild) {
   if (!e) return fail(SRE_ERR_INVALID, "null engine");
   if (!e->built) return fail(SRE_ERR_NOT_READY, "update before the first rebuild");
   HIP_TRY(hipSetDevice(e->device));
-  launch_update_positions(e->n_atoms, e->d_inv_perm, const_cast<float *>(e->d_pos),
-                          e->pos_stride, e->d_reps, rep0(e), e->d_pos4, e->d_backup,
-                          e->d_res4, e->d_skin_part, nullptr, e->stream);
+  enqueue_refresh(e, need_rebuild != nullptr);
   HIP_TRY(hipGetLastError());
   e->stats_valid = e->forces_valid = e->atom_stats_valid = false;
   if (need_rebuild) {
-    launch_rebuild_info(0, nullptr, nullptr, skin_part_count(e->n_atoms),
-                        e->d_skin_part, 0, e->d_flags, e->stream, nullptr, nullptr, 0,
-                        e->d_info_slices);
-    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(e->stream));
     const float d2 = skin_disp2(e);
     const float half = 0.5f * e->skin;
@@ -2605,13 +2615,11 @@ extern "C" sre_status sre_md_run(sre_engine *e, int n_steps, int rebuild_every,
   if (e->built) {
     // the bound positions may have been changed since the last step:
     // refresh the lattice copy and rebuild if they moved beyond skin/2
-    launch_update_positions(e->n_atoms, e->d_inv_perm,
-                            const_cast<float *>(e->d_pos), e->pos_stride,
-                            e->d_reps, rep0(e), e->d_pos4, e->d_backup, e->d_res4,
-                            e->d_skin_part, nullptr, e->stream);
+    enqueue_refresh(e, true);
     HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(e->stream));
     bool ok;
-    s = md_skin_ok(e, &ok);
+    s = md_skin_verdict(e, &ok);
     if (s != SRE_OK) return s;
     fresh = !ok;
   }

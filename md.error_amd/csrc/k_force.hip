@@ -31,7 +31,8 @@ __global__ __launch_bounds__(256) void k_update_positions(
     int n, const uint32_t *__restrict__ inv_perm, float *__restrict__ pos,
     int stride, const RepInfo *__restrict__ reps, Geom g1, int one_rep,
     uint4 *__restrict__ pos4, const uint4 *__restrict__ backup,
-    float4 *__restrict__ res4, float *__restrict__ skin_part, PerturbArgs pert) {
+    float4 *__restrict__ res4, float *__restrict__ skin_part, PerturbArgs pert,
+    SkinNow now) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int w = i / kWave;  // slots exist for the waves holding atoms
   const bool wslot = w * kWave < n;
@@ -73,7 +74,37 @@ __global__ __launch_bounds__(256) void k_update_positions(
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1)
     d2 = fmaxf(d2, __shfl_xor(d2, o, kWave));
-  if ((threadIdx.x & (kWave - 1)) == 0 && wslot && d2 > prev) skin_part[w] = d2;
+  const bool grew = (threadIdx.x & (kWave - 1)) == 0 && wslot && d2 > prev;
+  if (!now.ticket) {
+    if (grew) skin_part[w] = d2;
+    return;
+  }
+  // the largest of all: by the last block to finish, from values stored and
+  // loaded past the XCDs' own caches and arrived before the ticket is drawn
+  __shared__ float red[256 / kWave];
+  __shared__ bool last;
+  if (grew)
+    __hip_atomic_store(skin_part + w, d2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(now.ticket, 1u, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
+  __syncthreads();
+  if (!last) return;
+  const int parts = (n + kWave - 1) / kWave;
+  float m = 0.f;
+  for (int k = threadIdx.x; k < parts; k += 256)
+    m = fmaxf(m, __hip_atomic_load(skin_part + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < 256 / kWave; ++q) m = fmaxf(m, red[q]);
+    *now.bits = __float_as_uint(m);
+    *now.ticket = 0u;
+  }
 }
 
 // ---------------------------------------- next-step refresh in a force launch --
@@ -168,14 +199,15 @@ __device__ __forceinline__ bool force_block(const ForceArgs &a, int *bid, int *n
 void launch_update_positions(int n, const uint32_t *inv_perm, float *pos,
                              int stride, const RepInfo *reps, const RepInfo *host_rep0,
                              uint4 *pos4, const uint4 *backup, float4 *res4,
-                             float *skin_part, const PerturbArgs *pert, hipStream_t st) {
+                             float *skin_part, const PerturbArgs *pert, hipStream_t st,
+                             const SkinNow &now) {
   if (n <= 0) return;
   PerturbArgs p{};
   if (pert) p = *pert;
   const Geom g = host_rep0 ? geom_of(*host_rep0) : Geom{};
   hipLaunchKernelGGL(k_update_positions, dim3((n + 255) / 256), dim3(256), 0,
                      st, n, inv_perm, pos, stride, reps, g, host_rep0 ? 1 : 0, pos4,
-                     backup, res4, skin_part, p);
+                     backup, res4, skin_part, p, now);
 }
 
 // ------------------------------------------------------- rebuild info --

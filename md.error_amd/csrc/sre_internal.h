@@ -512,6 +512,16 @@ void launch_md_drift(int n, const uint32_t *inv_perm, float *pos, int stride,
                      const DriftArgs &drift, hipStream_t st);
 void launch_md_finish(int n, const double *part, MDState *state, float *vel,
                       hipStream_t st);
+// The largest displacement^2 since the last rebuild (float bits) from the refresh
+// itself: its last block reduces skin_part into *bits.  ticket: a word that is
+// zero before and after, or NULL for none of this.
+struct SkinNow {
+  unsigned *ticket = nullptr, *bits = nullptr;
+};
+// worth it up to this many atoms, one ticket per 256 (a refresh and the host's
+// answer, a launch for the largest / folded: 17.5 / 14.6 us at 4 000 atoms, 18.3
+// / 15.0 at 16 000, 18.9 / 17.8 at 64 000, 18.5 / 20.8 at 130 000)
+constexpr int kSkinFoldAtoms = 65536;
 // Position refresh + skin test: each wavefront keeps the largest squared
 // displacement it has seen since the last rebuild in skin_part[wave]
 // (skin_part_count(n) entries).
@@ -521,7 +531,8 @@ inline int skin_part_count(int n) { return (n + kWave - 1) / kWave; }
 void launch_update_positions(int n, const uint32_t *inv_perm, float *pos,
                              int stride, const RepInfo *reps, const RepInfo *host_rep0,
                              uint4 *pos4, const uint4 *backup, float4 *res4,
-                             float *skin_part, const PerturbArgs *pert, hipStream_t st);
+                             float *skin_part, const PerturbArgs *pert, hipStream_t st,
+                             const SkinNow &now = SkinNow{});
 
 // The next step's position refresh folded into a force launch (perturbation
 // mode, no integrator): n_blocks blocks in front of the force blocks
