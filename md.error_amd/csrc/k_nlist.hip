@@ -206,7 +206,7 @@ k_build_list(int n, const uint4 *__restrict__ pos4, const float *__restrict__ rc
       };
       // may some list pass its capacity with `more` further candidates?  longest
       // is an upper bound of the lists' lengths, made exact only when it is
-      // near the capacity
+      // near the capacity (so it takes in every chunk, whichever way it is tested)
       auto near_cap = [&](int more) {
         if (longest + more > cap) {
           longest = cnt[0];
@@ -337,7 +337,8 @@ k_build_list(int n, const uint4 *__restrict__ pos4, const float *__restrict__ rc
             float near = fabsf(dg[0][0]);
 #pragma unroll
             for (int r = 1; r < M; ++r) near = fminf(near, fabsf(dg[r / 4][r & 3]));
-            if (!(ballot64(near < band) || near_cap(q.filled))) {
+            const bool full = near_cap(q.filled);
+            if (!full && !ballot64(near < band)) {
               if (ballot64((unsigned)(q.j - s0) < (unsigned)M)) {   // the wave's own atoms
 #pragma unroll
                 for (int r = 0; r < M; ++r)
