@@ -1033,7 +1033,7 @@ constexpr uint64_t kNotYet = ~0ull;
 // is no longer kNotYet).
 static hipError_t launch_rebuild(sre_engine *e, hipGraphExec_t exec, const uint64_t **entry) {
   uint64_t *dst = e->h_log + 3 * (size_t)(e->log_launches % kRebuildLog);
-  *static_cast<volatile uint64_t *>(dst + 2) = kNotYet;
+  __atomic_store_n(dst + 2, kNotYet, __ATOMIC_RELEASE);
   hipError_t r = hipGraphLaunch(exec, e->stream);
   if (r != hipSuccess) return r;
   *entry = dst;
@@ -1153,8 +1153,11 @@ static sre_status do_rebuild(sre_engine *e) {
 // Waits until the queued rebuild of this log entry has written the largest
 // displacement^2 of the steps before it, which is its first launch's work.
 static sre_status wait_disp2(sre_engine *e, const uint64_t *info, float *d2) {
-  const volatile uint64_t *w = info + 2;
-  for (unsigned k = 1; *w == kNotYet; ++k) {
+  // (acquire: the log words and the range flag that the stream wrote before
+  // this one are read after it)
+  uint64_t w;
+  auto pending = [&] { return (w = __atomic_load_n(info + 2, __ATOMIC_ACQUIRE)) == kNotYet; };
+  for (unsigned k = 1; pending(); ++k) {
     if (k % 4096 != 0) {
       __builtin_ia32_pause();
       continue;
@@ -1166,9 +1169,9 @@ static sre_status wait_disp2(sre_engine *e, const uint64_t *info, float *d2) {
       continue;
     }
     if (r != hipSuccess) return fail(SRE_ERR_HIP, "rebuild: %s", hipGetErrorString(r));
-    if (*w == kNotYet) return fail(SRE_ERR_HIP, "rebuild: no displacement in the log");
+    if (pending()) return fail(SRE_ERR_HIP, "rebuild: no displacement in the log");
   }
-  const unsigned bits = (unsigned)(*w & 0xffffffffu);
+  const unsigned bits = (unsigned)(w & 0xffffffffu);
   memcpy(d2, &bits, sizeof(float));
   return SRE_OK;
 }
