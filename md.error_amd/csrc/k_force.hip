@@ -502,7 +502,10 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const PairParam *
   // eval_group.
   const unsigned nmax = (unsigned)(a.n - 1);
   const int per = W > 1 ? (groups + W - 1) / W : groups;
-  const int g0 = W > 1 ? part * per : 0, g1 = W > 1 ? min(groups, g0 + per) : groups;
+  // (a part without groups stays at the last one's rows and evaluates none)
+  const int first = part * per;
+  const int g0 = W > 1 ? min(first, max(groups - 1, 0)) : 0;
+  const int g1 = W > 1 ? (first < groups ? min(groups, first + per) : g0) : groups;
   auto prefetch = [&](uint4 *p, int *jr, int g) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
