@@ -894,8 +894,9 @@ __device__ __forceinline__ void pair_fp64(double dx, double dy, double dz, bool 
                                           double &wz) {
   const double d2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
   // coincident atoms: an infinite energy, as of a division (nonzero d2 is
-  // above 1e-90, the squares of the residuals' smallest steps)
-  const double ri2 = in ? rcp64(fmax(d2, 1e-200)) : 0.0;
+  // above 1e-90, the squares of the residuals' smallest steps: the sum is d2
+  // itself); a d2 that is no number stays none
+  const double ri2 = in ? rcp64(d2 + 1e-200) : 0.0;
   const double ri6 = ri2 * ri2 * ri2;
   const double fs = ri2 * ri6 * __builtin_fma(-P.A12, ri6, P.B6);
   fx = __builtin_fma(fs, dx, fx);
