@@ -794,20 +794,21 @@ extern "C" sre_status sre_arc_create(sre_arc **out, const double box[3],
     HIP_TRY(dalloc(&a->d_counts, nele));
     HIP_TRY(dalloc(&a->d_rho, nele));
     HIP_TRY(dalloc(&a->d_rhok, nele));
-    HIP_TRY(dalloc(&a->d_zr, nele));
     HIP_TRY(dalloc(&a->d_idx, nele));
     HIP_TRY(dalloc(&a->d_idx2, nele));
     HIP_TRY(dalloc(&a->d_rc, nele));
     HIP_TRY(dalloc(&a->d_res_err, nele));
     HIP_TRY(dalloc(&a->d_psum, (size_t)3 * arc_blocks(nele)));
-    for (int d = 0; d < 3; ++d)
+    a->matrix = true;
+    for (int d = 0; d < 3; ++d) a->matrix &= a->g.n[d] <= kArcAxisMax;
+    // of the direct transforms, without the matrix form
+    if (!a->matrix) HIP_TRY(dalloc(&a->d_zr, nele));
+    for (int d = 0; !a->matrix && d < 3; ++d)
       for (int dir = 0; dir < 2; ++dir) {
         HIP_TRY(dalloc(&a->d_tw[d][dir], a->g.n[d]));
         hipLaunchKernelGGL(k_arc_twiddle, dim3(arc_blocks(a->g.n[d])), dim3(kArcBlock),
                            0, a->stream, a->g.n[d], dir == 0 ? -1 : 1, a->d_tw[d][dir]);
       }
-    a->matrix = true;
-    for (int d = 0; d < 3; ++d) a->matrix &= a->g.n[d] <= kArcAxisMax;
     for (int d = 0; a->matrix && d < 3; ++d) {
       const int n = a->g.n[d], kt = arc_kt(n), jt = arc_jt(n);
       const size_t m = (size_t)kt * jt * kWave;
