@@ -566,10 +566,10 @@ struct NextRefresh {
 // place[i] = count[key]++ as k_cell_count.
 struct CountFold {
   int n_blocks;                // 0 = none; else a multiple of 8
-  const float *pos;            // caller positions
   int stride;
-  const int *rep_of;
   int n_cells;
+  const float *pos;            // caller positions
+  const int *rep_of;
   uint32_t *keys, *place, *count;
 };
 
@@ -577,6 +577,7 @@ struct ForceArgs {
   int n;
   int n_types;
   int cap;
+  int n_simd;                  // of the device (0: no launch that depends on it)
   const uint4 *pos4;
   const float4 *res4;          // FP64 form: sub-lattice residuals (sorted order)
   const float *rcut;
@@ -593,7 +594,6 @@ struct ForceArgs {
   double *fxd, *fyd, *fzd;     // FP64 output (sorted order)
   double *atom_stats;          // optional per-atom (E, Wxx, Wyy, Wzz)
   unsigned *err_flag;
-  int n_simd;          // of the device (0: no launch that depends on it)
   // perturbation step counter: one thread writes *ctr_out = *ctr_in + 1
   // (ctr_in == ctr_out, or two slots when the launch refreshes the next
   // step from *ctr_in); NULL = none
@@ -608,6 +608,11 @@ struct ForceArgs {
   NextRefresh next;            // the next step's refresh (perturbation mode)
   CountFold count;             // the next rebuild's cell histogram, or none
 };
+// A wavefront starts with scalar loads of its arguments and of the grid and
+// block sizes, which follow them; each further 64-byte line of those is a miss
+// of 0.25 us (with 456 bytes the sizes lay in one of their own: 9.77 us per
+// launch on a 64 000-atom slab and 6.20 at 8 000, with 440 9.50 and 5.96).
+static_assert(sizeof(ForceArgs) <= 440, "the sizes behind start another line");
 // The cell-window form of the mixed force evaluation (no list): tiles of
 // up to kCellTile sorted atoms of one cell column (tile_off / tiles_per_col
 // from launch_tile_map after the rebuild), kWave / kCellTile lanes per atom,
