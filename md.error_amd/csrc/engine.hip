@@ -119,7 +119,8 @@ struct sre_engine {
   int *d_start = nullptr;
   int start_cap = 0;
   int n_cols = 0;                  // (x, y) cell columns over all replicas
-  bool build_images = false;       // list build over second images (build_needs_images)
+  BuildForm build_form = BuildForm::kTiles;   // of the list build
+  bool dense = false;              // for it: long lists since the system was set
   uint32_t *d_tiles_per_col = nullptr, *d_tile_off = nullptr, *d_tile_tmp = nullptr;
   int tile_cap = 0;
   uint4 *d_pos4 = nullptr, *d_backup = nullptr;  // backup: caller order
@@ -522,6 +523,8 @@ extern "C" sre_status sre_set_system(sre_engine *e, int n_replicas,
   e->rc_dirty = true;
   e->tail_dirty = true;
   e->built = false;
+  e->max_count = 0;
+  e->dense = false;
   e->system_set = true;
   e->d_pos = nullptr;
   e->stats_valid = e->forces_valid = e->atom_stats_valid = false;
@@ -776,7 +779,6 @@ static sre_status prepare_tables(sre_engine *e) {
   }
   // cell grids
   long long cells = 0, cols = 0;
-  e->build_images = false;
   for (int r = 0; r < e->n_rep; ++r) {
     RepInfo &R = e->reps[r];
     const float rlmax = R.rc_max + e->skin;
@@ -786,12 +788,13 @@ static sre_status prepare_tables(sre_engine *e) {
                     "replica %d: rc_max + skin = %g is not below half the box "
                     "edge %d (%g)", r, rlmax, d, R.L[d]);
     choose_cell_grid(R, e->skin, e->tune.cell_xy, e->tune.cell_z);
-    e->build_images |= build_needs_images(R, e->skin);
     R.cell_off = (int)cells;
     R.col_off = (int)cols;
     cells += (long long)R.nc[0] * R.nc[1] * R.nc[2];
     cols += (long long)R.nc[0] * R.nc[1];
   }
+  e->dense |= e->max_count > kSparseLongest;
+  e->build_form = build_form(e->reps.data(), e->n_rep, e->skin, e->dense);
   if (cells >= (1ll << 31) - 2)
     return fail(SRE_ERR_CELL, "cell grid too large (%lld cells)", cells);
   e->n_cells = (int)cells;
@@ -939,7 +942,7 @@ static std::vector<unsigned char> rebuild_signature(const sre_engine *e,
                       e->tune.force_mode,
                       e->tune.force_lanes, e->n_types, e->pos_stride, n_parts,
                       (e->tail_bins > 0 && e->tail_mode == SRE_TAIL_EXACT) ? 1 : 0,
-                      e->rc_explicit ? 1 : 0, e->build_images ? 1 : 0};
+                      e->rc_explicit ? 1 : 0, (int)e->build_form};
   put(ints, sizeof ints);
   put(&e->skin, sizeof e->skin);
   const void *ptrs[] = {e->d_pos, e->d_rep_of, e->d_reps, e->sb.key_a, e->sb.key_b,
@@ -972,7 +975,7 @@ static void enqueue_build(sre_engine *e, hipStream_t st) {
                        e->d_list, e->d_nnb, e->d_build_part, e->d_tiles_per_col,
                        e->d_tile_off, e->d_tile_tmp, st);
   else
-    launch_build_list(e->tune.force_lanes, e->build_images, N, e->d_pos4,
+    launch_build_list(e->tune.force_lanes, e->build_form, N, e->d_pos4,
                       e->d_rcut, e->d_reps, e->d_start, e->skin, e->cap,
                       e->d_list, e->list_size, e->d_nnb, e->d_build_part, st);
 }

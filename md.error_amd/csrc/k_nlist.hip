@@ -17,7 +17,7 @@
 // ascending within a run), whatever the window was.  Entries go to the
 // wave-tiled column-major layout the force kernel reads (list_slot()).
 // Writes beyond the capacity are dropped but still counted; the host regrows
-// and rebuilds.
+// and rebuilds.  (Large dilute systems: a window per atom, the same lists.)
 //
 // The distance test is |x_i|^2 - rl_i^2 - 2 x_i.x_j + |x_j|^2 < 0 on
 // coordinates relative to the tile's centre, a contraction over (x, y, z, 1)
@@ -56,16 +56,20 @@ __device__ __forceinline__ float lane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// What bounds it: VALU issue (76 % busy at 2 million atoms, 145 instructions
+// What bounds it: VALU issue (79 % busy at 2 million atoms, 145 instructions
 // per atom; a form with one atom per 4 lanes and a divergent cursor over its
 // own windows took 240), and below ~100 000 atoms the length of the heaviest
 // wavefronts.  Per 64 candidates, 12 instructions form the local coordinates
 // for all M atoms, and each atom takes a compare of the matrix result and,
 // when lanes were accepted, the mask count (2), the slot (3) and the store.
 // Measured, M as chosen below, before -> now: 4 000 atoms (uniform cutoff)
-// 31 -> 15.4 us, 16 000 atoms with lists of 1 350 (IMG) 237 -> 128 us, 62 500
-// (slab) 52 -> 39.7 us, 2 048 000 (rc 2.5 to 6, 140 million entries, 0.56 GB
-// written) 1 000 -> 628 us.  M = 16 (fewer, longer wavefronts) was slower at
+// 31 -> 16 us, 16 000 atoms with lists of 1 350 (IMG) 228 -> 125 us, 62 500
+// (slab) 53 -> 39.4 us, 2 048 000 (rc 2.5 to 6, 140 million entries, 0.56 GB
+// written) 1 004 -> 615 us; boxes little wider than twice the list radius,
+// where chunks take the exact predicate, are faster too (a rebuild of 4 097
+// atoms in a cube of 16, rc 2.5: 71 -> 49 us; 3 000, rc 7.5: 166 -> 113).  Large
+// dilute systems are not, and keep a window per atom (k_build_list_sparse).
+// M = 16 (fewer, longer wavefronts) was slower at
 // every size.  Register budgets: seven (M = 4), six (M = 8) and four (IMG)
 // wavefronts per SIMD; eight spill scalar registers into vector lanes.
 template <int M, int TF, bool IMG>
@@ -407,6 +411,254 @@ k_build_list(int n, const uint4 *__restrict__ pos4, const float *__restrict__ rc
   }
 }
 
+// ---------------------------------------------------------- sparse build --
+//
+// The same lists, entry for entry, with a group of four lanes per atom and a
+// window of each atom's own: in a dilute gas the atoms of a tile lie far apart
+// along their column, and the window of all of them holds many times the
+// candidates of each (build_form: where the line lies).  Lane l of a group sets
+// up kSparseCols of the (x, y) columns that meet the sphere at a time: one or
+// two runs each, whose bounds are loaded together; a prefix sum over the group
+// turns the runs into one flat candidate sequence in LDS, of which the group
+// takes kSparseUnroll candidates per lane and round, the next round's gathers
+// in flight.  What bounds it: VALU issue, 74 instructions per atom where the
+// tiles take 108 (250 000 atoms, 0.02 per unit volume, cutoff 2.5).
+constexpr int kSparseLanes = 4;
+constexpr int kSparseCols = 4;     // columns per lane per chunk
+constexpr int kSparseUnroll = 6;   // candidates per lane per round
+
+__device__ __forceinline__ int sparse_max(int v) {
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, kWave));
+  return v;
+}
+
+__global__ __launch_bounds__(kBuildBlock) void k_build_list_sparse(
+    int n, int n_parts, int TF, const uint4 *__restrict__ pos4,
+    const float *__restrict__ rcut, const RepInfo *__restrict__ reps,
+    const int *__restrict__ start, float skin, int cap, int *__restrict__ list,
+    int *__restrict__ nnb, int2 *__restrict__ part) {
+  constexpr int TB = kSparseLanes, A = kWave / TB;
+  constexpr int CC = kSparseCols * TB;   // columns per chunk
+  constexpr int NS = 2 * CC;            // runs per chunk
+  constexpr int U = kSparseUnroll;
+  __shared__ int s_p0[kBuildBlock / TB][NS];    // first sorted atom of each run
+  __shared__ int s_end[kBuildBlock / TB][NS];   // inclusive prefix of run lengths
+  const int lane = threadIdx.x & (kWave - 1);
+  const int g = lane / TB, l = lane % TB;
+  const int gb = threadIdx.x / TB;
+  const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const int s = wave * A + g;
+  const bool act = s < n;
+  const int si = act ? s : n - 1;
+
+  const uint4 pi = pos4[si];
+  const __amdgpu_buffer_rsrc_t prs = pos_rsrc_idx(pos4, n);
+  const RepInfo &R = reps[pi.w >> 8];
+  const float qx = R.q[0], qy = R.q[1], qz = R.q[2];
+  const int ncx = R.nc[0], ncy = R.nc[1], ncz = R.nc[2];
+  const float hx = R.h[0], hy = R.h[1], hz = R.h[2];
+  const float ihz = 1.f / hz;
+  const float rl = rcut[si] + skin;
+  const float rl2 = rl * rl;
+  const float rlm = rl * 1.0001f + 1e-4f;  // conservative window radius
+  const float rlm2 = rlm * rlm;
+  const int cx = cell_of(pi.x, ncx), cy = cell_of(pi.y, ncy),
+            cz = cell_of(pi.z, ncz);
+  // position inside the own cell from the low 32 bits of u * nc
+  const float fx = (float)(uint32_t)((uint64_t)pi.x * (uint64_t)ncx) * (hx * 0x1p-32f);
+  const float fy = (float)(uint32_t)((uint64_t)pi.y * (uint64_t)ncy) * (hy * 0x1p-32f);
+  const float fz = (float)(uint32_t)((uint64_t)pi.z * (uint64_t)ncz) * (hz * 0x1p-32f);
+  const int kx = (int)ceilf(rlm / hx), ky = (int)ceilf(rlm / hy),
+            kz = (int)ceilf(rlm / hz);
+  const bool fullx = 2 * kx + 1 >= ncx, fully = 2 * ky + 1 >= ncy,
+             fullz = 2 * kz + 1 >= ncz;
+  const int ox0 = fullx ? -cx : -kx, ox1 = fullx ? ncx - 1 - cx : kx;
+  const int oy0 = fully ? -cy : -ky, oy1 = fully ? ncy - 1 - cy : ky;
+  const int noy = oy1 - oy0 + 1;
+  const int ncol = act ? (ox1 - ox0 + 1) * noy : 0;
+  const int ncol_w = __builtin_amdgcn_readfirstlane(sparse_max(ncol));
+
+  // list slots of this atom in the force kernel's layout (T = TF lanes):
+  // slot(k) = sbase + (k / TF) * 64 + k % TF, TF a power of two
+  const int AF = kWave / TF;
+  const int lt = __builtin_ctz((unsigned)TF);
+  const size_t sbase =
+      (size_t)(si / AF) * (size_t)cap * (size_t)AF + (size_t)((si % AF) * TF);
+  int *const lrow = list + sbase;
+  int *const sp0 = s_p0[gb];
+  int *const send = s_end[gb];
+  int count = 0;
+  for (int cbase = 0; cbase < ncol_w; cbase += CC) {
+    // runs of this lane's kSparseCols columns -> (first atom, length) in LDS
+    const int slot0 = l * 2 * kSparseCols;
+    int tot = 0;
+    // this lane's first column; the following ones step oy, then ox
+    int c = cbase + l * kSparseCols;
+    int ox = ox0 + c / noy, oy = oy0 + c % noy;
+#pragma unroll 2
+    for (int m = 0; m < kSparseCols; ++m, ++c) {
+      int ra0 = 0, rb0 = -1, ra1 = 0, rb1 = -1, colbase = 0;
+      if (c < ncol) {
+        float gx = 0.f, gy = 0.f;
+        if (!fullx) gx = ox > 0 ? ox * hx - fx : (ox < 0 ? fx + (-ox - 1) * hx : 0.f);
+        if (!fully) gy = oy > 0 ? oy * hy - fy : (oy < 0 ? fy + (-oy - 1) * hy : 0.f);
+        gx = fmaxf(gx, 0.f);
+        gy = fmaxf(gy, 0.f);
+        const float gxy2 = gx * gx + gy * gy;
+        if (gxy2 < rlm2) {
+          int cxw = cx + ox;
+          cxw += cxw < 0 ? ncx : 0;
+          cxw -= cxw >= ncx ? ncx : 0;
+          int cyw = cy + oy;
+          cyw += cyw < 0 ? ncy : 0;
+          cyw -= cyw >= ncy ? ncy : 0;
+          colbase = R.cell_off + (cxw * ncy + cyw) * ncz;
+          rb0 = ncz - 1;  // whole column unless the chord is shorter
+          if (!fullz) {
+            // (the window radius carries a 1e-4 margin, far above the
+            // rounding of a multiplication by 1/hz)
+            const float dz = sqrtf(fmaxf(rlm2 - gxy2, 0.f));
+            const int lo = cz + (int)floorf((fz - dz) * ihz);
+            const int hi = cz + (int)floorf((fz + dz) * ihz);
+            if (hi - lo + 1 < ncz) {
+              if (lo < 0) {
+                ra0 = lo + ncz; rb0 = ncz - 1; ra1 = 0; rb1 = hi;
+              } else if (hi >= ncz) {
+                ra0 = lo; rb0 = ncz - 1; ra1 = 0; rb1 = hi - ncz;
+              } else {
+                ra0 = lo; rb0 = hi;
+              }
+            }
+          }
+        }
+      }
+      const int b0 = rb0 >= ra0 ? start[colbase + ra0] : 0;
+      const int e0 = rb0 >= ra0 ? start[colbase + rb0 + 1] : 0;
+      const int b1 = rb1 >= ra1 ? start[colbase + ra1] : 0;
+      const int e1 = rb1 >= ra1 ? start[colbase + rb1 + 1] : 0;
+      // runs lie inside [0, n) by construction; the clamps keep every gather
+      // in bounds whatever the cell offsets hold
+      const int q0 = min(max(b0, 0), n), q1 = min(max(b1, 0), n);
+      const int n0 = max(min(e0, n) - q0, 0), n1 = max(min(e1, n) - q1, 0);
+      sp0[slot0 + 2 * m] = q0;
+      send[slot0 + 2 * m] = n0;       // length for now, prefix below
+      sp0[slot0 + 2 * m + 1] = q1;
+      send[slot0 + 2 * m + 1] = n1;
+      if (++oy > oy1) {
+        oy = oy0;
+        ++ox;
+      }
+      tot += n0 + n1;
+    }
+    // flat sequence: prefix over the group (lane-major slot order)
+    int incl = tot;
+#pragma unroll
+    for (int o = 1; o < TB; o <<= 1) {
+      const int t = __shfl_up(incl, o, TB);
+      if (l >= o) incl += t;
+    }
+    const int T = __shfl(incl, TB - 1, TB);
+    int run = incl - tot;
+    for (int r = 0; r < 2 * kSparseCols; ++r) {
+      run += send[slot0 + r];
+      send[slot0 + r] = run;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // stream the flat sequence: in round k0 lane l takes the U consecutive
+    // candidates v = (k0 TB + l) U + u
+    const int rounds = __builtin_amdgcn_readfirstlane(sparse_max((T + TB * U - 1) / (TB * U)));
+    // cursor over the runs: run cur covers flat indices [send[cur-1],
+    // end) and candidate v of it is sorted atom off + v (kept in registers;
+    // LDS is read only when the cursor moves to the next run)
+    int cur = 0, end = send[0], off = sp0[0];
+    // candidates of round k0 and their gathers (a lane past the sequence
+    // takes its own atom si, which the self test below rejects)
+    auto load = [&](int k0, int *jj, uint4 *cj) {
+      const int v0 = (k0 * TB + l) * U;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int v = v0 + u;
+        int j = si;
+        if (v < T) {
+          while (v >= end) {
+            ++cur;
+            const int b = end;
+            end = send[cur];
+            off = sp0[cur] - b;
+          }
+          j = off + v;
+        }
+        jj[u] = j;
+        cj[u] = gather_pos_idx<false>(prs, j);
+      }
+      asm volatile("" ::: "memory");
+    };
+    // the accepted candidates of a round, placed in flat-sequence order
+    // (lane by lane, each lane's U candidates in turn: an exclusive prefix
+    // of the lanes' accepted counts over the group), so that consecutive
+    // list entries are consecutive candidates -- neighbouring atoms of one
+    // cell column -- and the force kernel's lanes of one atom gather from
+    // the same few cache lines
+    auto accept = [&](const int *jj, const uint4 *cj) {
+      bool ok[U];
+      int c = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float dx = disp(cj[u].x, pi.x, qx);
+        const float dy = disp(cj[u].y, pi.y, qy);
+        const float dz2 = disp(cj[u].z, pi.z, qz);
+        // (an inactive group, s >= n, has no candidates: all its lanes
+        // hold j = si)
+        ok[u] = (jj[u] != si) & (dist2(dx, dy, dz2) < rl2);
+        c += ok[u] ? 1 : 0;
+      }
+      int incl = c;
+#pragma unroll
+      for (int o = 1; o < TB; o <<= 1) {
+        const int t = __shfl_up(incl, o, TB);
+        if (l >= o) incl += t;
+      }
+      int k = count + incl - c;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (ok[u] && k < cap) lrow[(unsigned)(((k >> lt) << 6) + (k & (TF - 1)))] = jj[u];
+        k += ok[u] ? 1 : 0;
+      }
+      count += __shfl(incl, TB - 1, TB);
+    };
+    // software pipeline: the gathers of round k0 + 1 are in flight while
+    // round k0 is tested; whole pairs of rounds in the loop (no branch in its
+    // body, so each gather is waited for only where it is used), the odd
+    // last round after it (every branch is wave-uniform)
+    int ja[U], jb[U];
+    uint4 ca[U], cb[U];
+    load(0, ja, ca);
+    int k0 = 0;
+    for (; k0 + 1 < rounds; k0 += 2) {
+      load(k0 + 1, jb, cb);
+      accept(ja, ca);
+      load(k0 + 2, ja, ca);
+      accept(jb, cb);
+    }
+    if (k0 < rounds) accept(ja, ca);
+    __builtin_amdgcn_wave_barrier();  // LDS reuse by the next chunk
+  }
+  // an overflowing list keeps its first cap entries (the partials below carry
+  // the full count, from which the host regrows), so no reader of the list
+  // ever runs past its rows
+  if (act && l == 0) nnb[s] = min(count, cap);
+  // this wave's longest list and total list length
+  int m = act ? count : 0;
+  int t = (act && l == 0) ? count : 0;
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    m = max(m, __shfl_xor(m, o, kWave));
+    t += __shfl_xor(t, o, kWave);
+  }
+  if (lane == 0 && wave < n_parts) part[wave] = make_int2(m, t);
+}
+
 int build_part_count(int mode, int n, int n_cols) {
   if (n <= 0) return 0;
   if (mode == 1) return (n + kWave - 1) / kWave + n_cols;  // tile grid
@@ -415,20 +667,47 @@ int build_part_count(int mode, int n, int n_cols) {
   return (n + per_block - 1) / per_block * (per_block / kBuildTile);
 }
 
-bool build_needs_images(const RepInfo &R, float skin) {
+static bool needs_images(const RepInfo &R, float skin) {
   const float rlm = (R.rc_max + skin) * 1.0001f + 1e-4f;
   for (int d = 0; d < 2; ++d)
     if (!(0.5001f * R.h[d] < 0.5f * R.L[d] - rlm)) return true;
   return false;
 }
 
+// Windows per atom where a rebuild is faster with them: in large dilute
+// systems.  x = list entries per atom at the mean density and the largest
+// cutoff; rebuild with tiles / with windows per atom, us, over uniform and
+// graded cutoffs of 2.5 to 5:
+//   16 000 atoms   x = 3.3  70.5 / 71.6    x = 12.5   71.3 / 76.2   x = 23   48.5 / 56.0
+//   40 000         x = 3.3  74.0 / 69.8    x = 12.5   85.3 / 82.6   x = 23   76.0 / 75.4
+//   120 000        x = 3.3 107.6 / 97.3    x = 12.5  140.8 / 125.3  x = 23  122.1 / 120.0
+//   600 000        x = 3.3 276.8 / 246.5   x = 12.5  392.5 / 347.7  x = 23  344.1 / 354.9
+//   1 500 000      x = 3.3 544.9 / 468.6   x = 12.5  822.4 / 715.2  x = 23  690.3 / 731.1
+// (at x = 18.4 within 5 % at every size).  A drop or a film in a large box has a
+// low mean too, but its lists are a liquid's, more than 60 entries: once such
+// lists have been met, tiles (a gas of 16 entries hardly has one of 40).
+BuildForm build_form(const RepInfo *reps, int n_rep, float skin, bool dense) {
+  double entries = 0.0, atoms = 0.0;
+  bool images = false;
+  for (int r = 0; r < n_rep; ++r) {
+    const RepInfo &R = reps[r];
+    const double rl = (double)R.rc_max + skin;
+    const double vol = (double)R.L[0] * R.L[1] * R.L[2];
+    atoms += R.n_atoms;
+    entries += 4.18879 * rl * rl * rl * R.n_atoms / vol * R.n_atoms;
+    images |= needs_images(R, skin);
+  }
+  if (!dense && atoms >= 40000.0 && entries < 16.0 * atoms) return BuildForm::kSparse;
+  return images ? BuildForm::kImages : BuildForm::kTiles;
+}
+
 template <int M, int TF>
-static void launch_build_m(bool images, int n, const uint4 *pos4, const float *rcut,
+static void launch_build_m(BuildForm form, int n, const uint4 *pos4, const float *rcut,
                            const RepInfo *reps, const int *start, float skin, int cap,
                            int *list, size_t list_len, int *nnb, int2 *part, hipStream_t st) {
   constexpr int most = kBuildWaves * 8;   // every part[] entry is written
   const dim3 g((n + most - 1) / most * (8 / M)), b(kBuildBlock);
-  if (images)
+  if (form == BuildForm::kImages)
     hipLaunchKernelGGL((k_build_list<M, TF, true>), g, b, 0, st, n, pos4, rcut, reps, start,
                        skin, cap, list, list_len, nnb, part);
   else
@@ -436,11 +715,18 @@ static void launch_build_m(bool images, int n, const uint4 *pos4, const float *r
                        skin, cap, list, list_len, nnb, part);
 }
 
-void launch_build_list(int force_lanes, bool images, int n, const uint4 *pos4,
+void launch_build_list(int force_lanes, BuildForm form, int n, const uint4 *pos4,
                        const float *rcut, const RepInfo *reps, const int *start,
                        float skin, int cap, int *list, size_t list_len, int *nnb,
                        int2 *part, hipStream_t st) {
   if (n <= 0) return;
+  if (form == BuildForm::kSparse) {
+    constexpr int per_block = kBuildBlock / kSparseLanes;
+    hipLaunchKernelGGL(k_build_list_sparse, dim3((n + per_block - 1) / per_block),
+                       dim3(kBuildBlock), 0, st, n, build_part_count(0, n, 0), force_lanes,
+                       pos4, rcut, reps, start, skin, cap, list, nnb, part);
+    return;
+  }
   // Four atoms per wavefront while eight leave the chip short of wavefronts
   // to even out the heavy ones (interface atoms): the list build alone takes
   // 15.4 against 19.0 us at 4 000 atoms (uniform cutoff) and 39.7 against
@@ -451,10 +737,10 @@ void launch_build_list(int force_lanes, bool images, int n, const uint4 *pos4,
 #define SRE_BUILD(TF)                                                                       \
   do {                                                                                      \
     if (few)                                                                                \
-      launch_build_m<4, TF>(images, n, pos4, rcut, reps, start, skin, cap, list, list_len,  \
+      launch_build_m<4, TF>(form, n, pos4, rcut, reps, start, skin, cap, list, list_len,  \
                             nnb, part, st);                                                 \
     else                                                                                    \
-      launch_build_m<8, TF>(images, n, pos4, rcut, reps, start, skin, cap, list, list_len,  \
+      launch_build_m<8, TF>(form, n, pos4, rcut, reps, start, skin, cap, list, list_len,  \
                             nnb, part, st);                                                 \
   } while (0)
   switch (force_lanes) {

@@ -387,10 +387,15 @@ void launch_assign_rc(int n, const float *pos, int stride, const int *rep_of,
 // (build_part_count entries, every one written by every launch; mode 0: one
 // pair per 16 sorted atoms); launch_rebuild_info reduces them.
 int build_part_count(int mode, int n, int n_cols);
-// images: some replica's cells are so large a part of its box that a tile's
-// atoms may see a candidate's second image along x or y (build_needs_images)
-bool build_needs_images(const RepInfo &R, float skin);
-void launch_build_list(int force_lanes, bool images, int n, const uint4 *pos4,
+// The form of mode 0 (same lists): tiles of atoms that share a window, such
+// tiles with candidates' second images along x and y (some replica's cells are
+// so large a part of its box that a tile's atoms may see them), or a window per
+// atom (k_nlist.hip: build_form).
+enum class BuildForm { kTiles, kImages, kSparse };
+// dense: lists longer than kSparseLongest have been met
+constexpr int kSparseLongest = 48;
+BuildForm build_form(const RepInfo *reps, int n_rep, float skin, bool dense);
+void launch_build_list(int force_lanes, BuildForm form, int n, const uint4 *pos4,
                        const float *rcut, const RepInfo *reps, const int *start,
                        float skin, int cap, int *list, size_t list_len, int *nnb,
                        int2 *part, hipStream_t st);

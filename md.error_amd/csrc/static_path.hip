@@ -266,8 +266,8 @@ extern "C" sre_status sre_forces_static(int n_atoms, const float *d_xyz, int str
                          d_reps, d_rc, n_types, d_start, d_pos4, d_backup, d_inv_perm,
                          nullptr, d_rcut, d_tail_idx, nullptr, st);
   }
-  launch_build_list(T, build_needs_images(R, skin), N, d_pos4, d_rcut, d_reps, d_start, skin, cap, d_list, list_len, d_nnb,
-                    d_build_part, st);
+  launch_build_list(T, build_form(&R, 1, skin, false), N, d_pos4, d_rcut, d_reps, d_start, skin, cap,
+                    d_list, list_len, d_nnb, d_build_part, st);
   launch_rebuild_info(n_parts, d_build_part, d_counters, 0, nullptr, 0, nullptr, st);
   HIP_TRY(hipGetLastError());
   uint64_t back[2];                  // the bad-type word and the longest list
