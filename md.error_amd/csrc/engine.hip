@@ -989,9 +989,13 @@ static void enqueue_build(sre_engine *e, hipStream_t st) {
 // 94.6 / 79.2 us at 64 000 atoms, 104.6 / 93.7 at 80 000, 126.8 / 115.0 at
 // 120 000 atoms in 23 000 cells, 156 / 161 at 200 000 in 39 000); beyond, the
 // radix sort's passes are cheaper than the scattered counts and the scan of
-// all of them by one block
+// all of them by one block, and so they are beyond 15 360 with many atoms per
+// cell, whose ranks take long (500 000 atoms, 25 per cell: 494.6 / 502.3 us,
+// 1.5 million, 65 per cell: 4290 / 4324; 300 000, 13 per cell: 229.8 / 230.2)
 static bool counting_sort(const sre_engine *e) {
-  return e->tune.sort_mode == 2 || (e->tune.sort_mode == 0 && e->n_cells <= kCountCells);
+  if (e->tune.sort_mode != 0) return e->tune.sort_mode == 2;
+  return e->n_cells <= kPlaceCells ||
+         (e->n_cells <= kCountCells && e->n_atoms <= 16ll * e->n_cells);
 }
 
 // counted: the cell histogram was made by the force launch just before
