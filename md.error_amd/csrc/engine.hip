@@ -1255,7 +1255,9 @@ static ForceArgs force_args(sre_engine *e, bool atom_stats) {
   // force kernel's waves with 4 lanes per atom
   a.wave_len = (e->tune.build_mode == 0 && e->list_lanes == 4) ? e->d_build_part : nullptr;
   a.xcd_remap = e->tune.xcd_remap;
-  a.n_simd = e->n_simd;
+  // eight groups of two rows per tile and more, of the longest list (both sides
+  // at k_force_mixed_rows); the sums do not depend on it
+  a.n_simd = e->max_count >= 16 * e->list_lanes ? e->n_simd : 0;
   a.has_shift = e->has_shift ? 1 : 0;
   // persistent launch: whole blocks of the tuned size
   const int per_block = e->tune.block / kWave;

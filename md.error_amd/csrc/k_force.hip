@@ -646,7 +646,10 @@ __global__ __launch_bounds__(256) void k_force_mixed(ForceArgs a) {
 // 4.6 / 4.2 at 4 000, 5.6 / 4.4 on an 8 000-atom slab, 5.6 / 5.2 at 16 000, 40.7
 // / 37.3 at 16 000 atoms with 1 366 list entries each; with two tiles per SIMD
 // 6.7 / 6.3 but 71.0 / 72.8 on such long lists, with four 8.9 / 9.9.  (2 and 8
-// wavefronts lie between or behind.)
+// wavefronts lie between or behind.)  With few groups in a tile the parts' start
+// costs more than they save: lists of about 2 entries 2.7 / 2.9 at 4 000 atoms
+// and 2.8 / 3.5 at 16 000, of 30 (four groups) 3.4 / 3.7 at 16 000, 80 entries
+// over 16 lanes (three) 3.7 / 4.4; so from eight groups in the longest list on.
 constexpr int kRowWaves = 4;
 template <int T, bool TAIL, bool MULTI>
 __global__ __launch_bounds__(kWave * kRowWaves) void k_force_mixed_rows(ForceArgs a) {
