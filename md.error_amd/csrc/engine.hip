@@ -1259,6 +1259,7 @@ static ForceArgs force_args(sre_engine *e, bool atom_stats) {
   // at k_force_mixed_rows); the sums do not depend on it
   a.n_simd = e->max_count >= 16 * e->list_lanes ? e->n_simd : 0;
   a.has_shift = e->has_shift ? 1 : 0;
+  a.short_lists = e->max_count <= std::max(10, 5 * e->list_lanes / 2) ? 1 : 0;
   // persistent launch: whole blocks of the tuned size
   const int per_block = e->tune.block / kWave;
   a.persist_waves = e->tune.persistent > 0

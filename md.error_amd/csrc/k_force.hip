@@ -923,7 +923,13 @@ __device__ __forceinline__ void pair_fp64(double dx, double dy, double dz, bool 
 // loads, per-lane trip count, correctly rounded division, separate multiply
 // and add) took 21.9 us on the 64k slab (8 lanes per atom, energy and virial),
 // 7.3 at 4 000 atoms and 280 at 1 million; this one 16.7, 5.1 and 221 us.
-template <int T, bool STATS, bool TAIL, bool MULTI, bool NEXT>
+// SHORT: a plain loop over each lane's own rows, with the same arithmetic in the
+// same order, where the longest list is no more than 10 entries or 2.5 rows: the
+// pipeline's start then costs more than it hides (64 000 atoms in a gas of 2
+// entries each, pipelined / plain: 5.1 / 4.3 us with 8 lanes, 3.8 / 3.3 with 4;
+// 300 000 with 7 entries 17.4 / 16.9, with energy and virial 23.7 / 21.7; with
+// 17 entries the pipelined one is ahead, 23.4 against 26.6).
+template <int T, bool STATS, bool TAIL, bool MULTI, bool NEXT, bool SHORT>
 __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
   if (a.ctr_out && blockIdx.x == 0 && threadIdx.x == 0) *a.ctr_out = *a.ctr_in + 1;
   __shared__ PairParamD sp[MULTI ? kMaxPairTypes : 1];
@@ -954,7 +960,6 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
   const int nn = act ? a.nnb[si] : 0;
   const int lim = nn - l;
   const int ti = (int)(pi.w & 0xffu) * a.n_types;
-  const int groups = __builtin_amdgcn_readfirstlane(wave_max_int((nn + T - 1) / T));
   PairParamD P = a.paramsd[0];
   const size_t tile0 = (size_t)__builtin_amdgcn_readfirstlane(wave) * (size_t)a.cap * A;
   const size_t lrem = a.list_len > tile0 ? a.list_len - tile0 : 0;
@@ -970,11 +975,13 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
       const_cast<float4 *>(a.res4), (short)16, a.n * 16, 0x00020000);
   double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
   struct Pj { uint4 p; float3 r; };
-  auto fetch = [&](Pj &q, int &jr, int g) {
-    const int j = g * T < lim ? jr : si;
+  auto gather = [&](Pj &q, int j) {
     q.p = gather_pos_idx<MULTI>(prs, j);
     const sre_u32x3 v = sre_struct_load_v3(rrs, j, 0, 0, 0);
     q.r = make_float3(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]));
+  };
+  auto fetch = [&](Pj &q, int &jr, int g) {
+    gather(q, g * T < lim ? jr : si);
     jr = row(g + 2);
     asm volatile("" ::: "memory");
   };
@@ -993,18 +1000,27 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
                                      (double)q.r.z - (double)ri.z);
     pair_fp64<STATS>(dx, dy, dz, in, P, fx, fy, fz, e, wx, wy, wz);
   };
-  int ja = row(0), jb = row(1);
-  asm volatile("" ::: "memory");
-  Pj qa, qb;
-  fetch(qa, ja, 0);
-  int g = 0;
-  for (; g + 1 < groups; g += 2) {
-    fetch(qb, jb, g + 1);
-    eval(qa, g);
-    fetch(qa, ja, g + 2);
-    eval(qb, g + 1);
+  if (SHORT) {     // each lane its own rows only
+    for (int g = 0; g * T < lim; ++g) {
+      Pj q;
+      gather(q, row(g));
+      eval(q, g);
+    }
+  } else {
+    const int groups = __builtin_amdgcn_readfirstlane(wave_max_int((nn + T - 1) / T));
+    int ja = row(0), jb = row(1);
+    asm volatile("" ::: "memory");
+    Pj qa, qb;
+    fetch(qa, ja, 0);
+    int g = 0;
+    for (; g + 1 < groups; g += 2) {
+      fetch(qb, jb, g + 1);
+      eval(qa, g);
+      fetch(qa, ja, g + 2);
+      eval(qb, g + 1);
+    }
+    if (g < groups) eval(qa, g);
   }
-  if (g < groups) eval(qa, g);
   fx = group_sum(fx, T);
   fy = group_sum(fy, T);
   fz = group_sum(fz, T);
@@ -1065,12 +1081,13 @@ static void launch_mixed_s(int grid, int block, bool multi, const ForceArgs &a,
 
 template <int T, bool STATS, bool TAIL, bool MULTI>
 static void launch_fp64_n(int grid, int block, const ForceArgs &a, hipStream_t st) {
+  const dim3 g(grid), b(block);
   if (a.next.active)
-    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, true>), dim3(grid), dim3(block), 0,
-                       st, a);
+    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, true, false>), g, b, 0, st, a);
+  else if (a.short_lists)
+    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, false, true>), g, b, 0, st, a);
   else
-    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, false>), dim3(grid), dim3(block), 0,
-                       st, a);
+    hipLaunchKernelGGL((k_force_fp64<T, STATS, TAIL, MULTI, false, false>), g, b, 0, st, a);
 }
 
 // the energy shift only enters the statistics

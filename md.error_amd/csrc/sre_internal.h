@@ -610,6 +610,7 @@ struct ForceArgs {
   int has_shift;               // some pair type has a nonzero energy shift
   int persist_waves;           // mixed form: > 0 = persistent launch of that many
                                // wavefronts, each taking a contiguous chunk of tiles
+  int short_lists;             // FP64 form: no list is long enough to pipeline
   NextRefresh next;            // the next step's refresh (perturbation mode)
   CountFold count;             // the next rebuild's cell histogram, or none
 };

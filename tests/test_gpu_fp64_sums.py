@@ -1,5 +1,6 @@
-"""The FP64 form's sums over whole lists (odd and even numbers of row groups,
-masked rows, partial tiles) against a float64 evaluation of the same pairs on
+"""The FP64 form's sums over whole lists (the pipelined loop: odd and even
+numbers of row groups, masked rows, partial tiles; and the loop of short lists,
+with empty ones) against a float64 evaluation of the same pairs on
 the host, and a coordinate that is no number."""
 import numpy as np
 import pytest
@@ -30,14 +31,16 @@ def engine(xyz, box, lanes, eps, sig, types, rc=RC):
 
 
 @pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16])
-@pytest.mark.parametrize("n,species", [(343, 1), (1327, 2), (4095, 1)])
-def test_list_sums_match_float64(torch_cuda, lanes, n, species):
+@pytest.mark.parametrize("n,species,spacing", [
+    (343, 1, 1.05), (1327, 2, 1.05), (4095, 1, 1.05),
+    (1327, 2, 1.9), (2001, 1, 2.4)])      # short lists: from 8 lanes on, for all lanes
+def test_list_sums_match_float64(torch_cuda, lanes, n, species, spacing):
     rng = np.random.default_rng(n)
     m = int(np.ceil(n ** (1.0 / 3.0)))
     xyz = np.zeros((n, 4), np.float32)
-    xyz[:, :3] = 1.05 * (np.stack(np.unravel_index(rng.permutation(m ** 3)[:n], (m, m, m)), 1)
-                         + 0.5 + rng.uniform(-0.06, 0.06, (n, 3)))
-    box = np.full(3, 1.05 * m, np.float32)
+    site = np.stack(np.unravel_index(rng.permutation(m ** 3)[:n], (m, m, m)), 1)
+    xyz[:, :3] = spacing * (site + 0.5 + rng.uniform(-0.06, 0.06, (n, 3)))
+    box = np.full(3, spacing * m, np.float32)
     types = (np.arange(n) % 3 % species).astype(np.int32)
     eps = np.array([[1.0, 0.75], [0.75, 0.5]], np.float32)[:species, :species]
     sig = np.array([[1.0, 0.875], [0.875, 0.75]], np.float32)[:species, :species]
