@@ -793,8 +793,6 @@ static sre_status prepare_tables(sre_engine *e) {
     cells += (long long)R.nc[0] * R.nc[1] * R.nc[2];
     cols += (long long)R.nc[0] * R.nc[1];
   }
-  e->dense |= e->max_count > kSparseLongest;
-  e->build_form = build_form(e->reps.data(), e->n_rep, e->skin, e->dense);
   if (cells >= (1ll << 31) - 2)
     return fail(SRE_ERR_CELL, "cell grid too large (%lld cells)", cells);
   e->n_cells = (int)cells;
@@ -873,9 +871,15 @@ static sre_status prepare_tables(sre_engine *e) {
     }
     e->graph_epoch++;
   }
-  if (e->reps_uploaded.size() != e->reps.size() ||
-      memcmp(e->reps_uploaded.data(), e->reps.data(),
-             sizeof(RepInfo) * e->reps.size()) != 0) {
+  const bool changed = e->reps_uploaded.size() != e->reps.size() ||
+                       memcmp(e->reps_uploaded.data(), e->reps.data(),
+                              sizeof(RepInfo) * e->reps.size()) != 0;
+  const bool dense = e->dense || e->max_count > kSparseLongest;
+  if (changed || dense != e->dense) {
+    e->dense = dense;
+    e->build_form = build_form(e->reps.data(), e->n_rep, e->skin, dense);
+  }
+  if (changed) {
     HIP_TRY(hipMemcpy(e->d_reps, e->reps.data(), sizeof(RepInfo) * e->n_rep,
                       hipMemcpyHostToDevice));
     e->reps_uploaded = e->reps;

@@ -17,7 +17,8 @@
 // ascending within a run), whatever the window was.  Entries go to the
 // wave-tiled column-major layout the force kernel reads (list_slot()).
 // Writes beyond the capacity are dropped but still counted; the host regrows
-// and rebuilds.  (Large dilute systems: a window per atom, the same lists.)
+// and rebuilds.  (Large dilute systems and batches of small boxes: a window
+// per atom, the same lists.)
 //
 // The distance test is |x_i|^2 - rl_i^2 - 2 x_i.x_j + |x_j|^2 < 0 on
 // coordinates relative to the tile's centre, a contraction over (x, y, z, 1)
@@ -26,12 +27,15 @@
 // pair whose value lies outside a band around 0 that bounds its rounding;
 // the rare pair inside the band is decided by the exact predicate, so the
 // pair set is the exact predicate's.
+#include <algorithm>
+
 #include "sre_internal.h"
 
 namespace sre {
 
 constexpr int kBuildBlock = 256;
 constexpr int kBuildTile = 16;    // atoms per entry of part[]
+constexpr int kTileAtoms = 80000; // atoms from which a tile has eight (launch_build_list)
 constexpr int kBuildWaves = kBuildBlock / kWave;
 
 typedef float sre_f32x4 __attribute__((ext_vector_type(4)));
@@ -66,9 +70,10 @@ __device__ __forceinline__ float lane_f(float v, int l) {
 // 31 -> 16 us, 16 000 atoms with lists of 1 350 (IMG) 228 -> 125 us, 62 500
 // (slab) 53 -> 39.4 us, 2 048 000 (rc 2.5 to 6, 140 million entries, 0.56 GB
 // written) 1 004 -> 615 us; boxes little wider than twice the list radius,
-// where chunks take the exact predicate, are faster too (a rebuild of 4 097
-// atoms in a cube of 16, rc 2.5: 71 -> 49 us; 3 000, rc 7.5: 166 -> 113).  Large
-// dilute systems are not, and keep a window per atom (k_build_list_sparse).
+// where chunks take the exact predicate, are faster too while few atoms fill the
+// chip (a rebuild of 3 000 atoms in a cube of 16, rc 7.5: 166 -> 113 us).  Large
+// dilute systems and batches of small boxes are not, and keep a window per atom
+// (k_build_list_sparse).
 // M = 16 (fewer, longer wavefronts) was slower at
 // every size.  Register budgets: seven (M = 4), six (M = 8) and four (IMG)
 // wavefronts per SIMD; eight spill scalar registers into vector lanes.
@@ -416,7 +421,8 @@ k_build_list(int n, const uint4 *__restrict__ pos4, const float *__restrict__ rc
 // The same lists, entry for entry, with a group of four lanes per atom and a
 // window of each atom's own: in a dilute gas the atoms of a tile lie far apart
 // along their column, and the window of all of them holds many times the
-// candidates of each (build_form: where the line lies).  Lane l of a group sets
+// candidates of each; and in boxes of two to three list radii tiles have much
+// to test or fall apart (build_form: where the lines lie).  Lane l of a group sets
 // up kSparseCols of the (x, y) columns that meet the sphere at a time: one or
 // two runs each, whose bounds are loaded together; a prefix sum over the group
 // turns the runs into one flat candidate sequence in LDS, of which the group
@@ -674,10 +680,10 @@ static bool needs_images(const RepInfo &R, float skin) {
   return false;
 }
 
-// Windows per atom where a rebuild is faster with them: in large dilute
-// systems.  x = list entries per atom at the mean density and the largest
-// cutoff; rebuild with tiles / with windows per atom, us, over uniform and
-// graded cutoffs of 2.5 to 5:
+// Windows per atom where a rebuild is faster with them, for most of the atoms of
+// a large system.  x = list entries per atom at the mean density and the
+// replica's largest cutoff; rebuild with tiles / with windows per atom, us.
+// (a) Dilute: x < 16 and 40 000 atoms (uniform and graded cutoffs of 2.5 to 5).
 //   16 000 atoms   x = 3.3  70.5 / 71.6    x = 12.5   71.3 / 76.2   x = 23   48.5 / 56.0
 //   40 000         x = 3.3  74.0 / 69.8    x = 12.5   85.3 / 82.6   x = 23   76.0 / 75.4
 //   120 000        x = 3.3 107.6 / 97.3    x = 12.5  140.8 / 125.3  x = 23  122.1 / 120.0
@@ -686,18 +692,46 @@ static bool needs_images(const RepInfo &R, float skin) {
 // (at x = 18.4 within 5 % at every size).  A drop or a film in a large box has a
 // low mean too, but its lists are a liquid's, more than 60 entries: once such
 // lists have been met, tiles (a gas of 16 entries hardly has one of 40).
+// (b) Boxes so short along z that a tile's window takes in the whole column
+// where its atoms' own do not, which has the tile done atom by atom (liquids in
+// cubes and plates of 2.9 list radii along z): x < 128 and 15 000 atoms, or
+// x < 300 and 20 000.
+//   cube / plate, x = 69 (cutoff 2.5)   16 000 atoms  66.1 / 54.1, 70.6 / 64.0
+//                                      100 000        255 / 96, 238 / 114
+//   x = 260   16 000  103.5 / 89.6, 105.8 / 109.7   100 000  377 / 198, 355 / 259
+//   (plate, x = 470   16 000  125 / 161   100 000  443 / 373   400 000  1149 / 1260)
+// (c) Boxes whose atoms see second images (x < 200), or so short along z that a
+// tile's pairs take the exact predicate (x < 500): 40 000 atoms.
+//   cube of 2.1 list radii, x = 69   24 000  50.2 / 46.7   65 000  72.9 / 61.7   400 000  259 / 208
+//   2.6 x 8 x 8 list radii, x = 69   24 000  56.3 / 61.1   65 000  85.8 / 77.0   400 000  314 / 279
+//   cube of 2.6, x = 113            400 000  357 / 297     x = 172   439 / 394   x = 260  514 / 510
+//   plate of 2.05, x = 69           400 000  328 / 305     x = 260   752 / 696   x = 470  1195 / 1050
+//   (plate of 2.35, x = 69          400 000  330 / 321     x = 260   583 / 746)
 BuildForm build_form(const RepInfo *reps, int n_rep, float skin, bool dense) {
-  double entries = 0.0, atoms = 0.0;
+  double atoms = 0.0, dilute = 0.0, whole = 0.0, small = 0.0;
   bool images = false;
+  for (int r = 0; r < n_rep; ++r) atoms += reps[r].n_atoms;
   for (int r = 0; r < n_rep; ++r) {
     const RepInfo &R = reps[r];
     const double rl = (double)R.rc_max + skin;
-    const double vol = (double)R.L[0] * R.L[1] * R.L[2];
-    atoms += R.n_atoms;
-    entries += 4.18879 * rl * rl * rl * R.n_atoms / vol * R.n_atoms;
-    images |= needs_images(R, skin);
+    const double rho = R.n_atoms / ((double)R.L[0] * R.L[1] * R.L[2]);
+    const double x = 4.18879 * rl * rl * rl * rho;
+    const bool second = needs_images(R, skin);
+    // a tile's length along its column: 4 or 8 atoms, or a cell, inside which
+    // they are in caller order
+    const double len = std::max((double)R.h[2], (atoms < kTileAtoms ? 4 : 8) /
+                                                    (rho * R.h[0] * R.h[1]));
+    const bool column = 2 * (int)ceil(rl / R.h[2]) + 1 < R.nc[2] &&
+                        (len + 2.0 * rl) / R.h[2] + 2.0 > R.nc[2];
+    const bool flat = 0.3 * R.h[2] > 0.5 * R.L[2] - rl;
+    if (x < 16.0 && !dense) dilute += R.n_atoms;
+    if (column && (x < 128.0 || (x < 300.0 && atoms >= 20000.0))) whole += R.n_atoms;
+    if ((second && x < 200.0) || (column && x < 300.0) || (flat && x < 500.0)) small += R.n_atoms;
+    images |= second;
   }
-  if (!dense && atoms >= 40000.0 && entries < 16.0 * atoms) return BuildForm::kSparse;
+  const double most = 0.5 * atoms;
+  if (atoms >= 40000.0 && (dilute > most || small > most)) return BuildForm::kSparse;
+  if (atoms >= 15000.0 && whole > most) return BuildForm::kSparse;
   return images ? BuildForm::kImages : BuildForm::kTiles;
 }
 
@@ -733,7 +767,7 @@ void launch_build_list(int force_lanes, BuildForm form, int n, const uint4 *pos4
   // 42.8 us at 62 500 (slab); at 90 000 a rebuild takes 127.0 against 124.3,
   // at 1 000 000 582 against 501 us, since eight share the candidates' local
   // coordinates and half as many tiles set up windows.
-  const bool few = n < 80000;
+  const bool few = n < kTileAtoms;
 #define SRE_BUILD(TF)                                                                       \
   do {                                                                                      \
     if (few)                                                                                \

@@ -1,8 +1,9 @@
-"""The list build of large dilute systems (a window per atom) against the
-oracle's pair sets and, entry for entry, against the build by tiles, which the
-same engine takes once it has met long lists: FP64 forces are summed in list
-order.  Both sides of the rule, remainders of a wavefront's atoms, whole-box
-windows, lists that outgrow their capacity, replicas."""
+"""The list build of large dilute systems and of batches of small boxes (a
+window per atom) against the oracle's pair sets and, entry for entry, against
+the build by tiles, which the same engine takes once it has met long lists, or a
+smaller batch: FP64 forces are summed in list order.  Both sides of the rule,
+remainders of a wavefront's atoms, whole-box windows, lists that outgrow their
+capacity, replicas."""
 import numpy as np
 import pytest
 
@@ -121,3 +122,62 @@ def test_replicas(torch_cuda):
         assert np.array_equal(o - o[0], off)
         assert np.array_equal(gj[o[0]:o[-1]] - first, j)
         first += len(x)
+
+
+# box, cutoff, replicas: columns that a tile's window fills, second images along
+# both or one of x and y, plates, replicas of which most atoms want it or do not
+BATCHES = [
+    [((8.1, 8.1, 8.1), 2.5, 46)],
+    [((6.1, 6.3, 5.9), 2.5, 360)],
+    [((7.3, 22.0, 22.0), 2.5, 18)],
+    [((16.8, 16.8, 5.75), 2.5, 38)],
+    [((11.0, 11.1, 11.05), 3.5, 21)],
+    [((8.1, 8.1, 8.1), 2.5, 40), ((14.0, 14.0, 14.0), 2.5, 3)],
+    [((8.1, 8.1, 8.1), 2.5, 20), ((14.0, 14.0, 14.0), 2.5, 6)],
+]
+
+
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+@pytest.mark.parametrize("lanes", [4, 16])
+def test_batches_of_small_boxes(torch_cuda, batch, lanes):
+    rng = np.random.default_rng(batch)
+    ns, boxes, xs, rc = [], [], [], 0.0
+    for box, rc, copies in BATCHES[batch]:
+        box = np.asarray(box, np.float32)
+        c = np.maximum(1, np.floor(box / 1.1)).astype(int)
+        for _ in range(copies):
+            n = int(np.prod(c)) - rng.integers(0, 9)
+            s = np.stack(np.unravel_index(rng.permutation(np.prod(c))[:n], c), 1)
+            x = np.zeros((n, 4), np.float32)
+            x[:, :3] = np.mod((s + 0.5 + rng.uniform(-0.07, 0.07, (n, 3))) * (box / c), box)
+            ns.append(n)
+            boxes.append(box)
+            xs.append(x)
+    table = np.full((1, 1, 1), rc, np.float32)
+
+    def run(which):
+        e = engine([ns[r] for r in which], np.array([boxes[r] for r in which]), table, "fp64", lanes)
+        e.upload_positions(np.concatenate([xs[r] for r in which]))
+        e.rebuild()
+        off, j = e.export_pairs()
+        e.compute(stats=True)
+        f, a = e.forces(), e.atom_stats()
+        e.close()
+        return off, j, f, a
+
+    R = len(ns)
+    off, j, f, a = run(range(R))
+    start = np.concatenate([[0], np.cumsum(ns)])
+    few = sorted({0, 1, R - 1})            # a batch of fewer than 15 000 atoms: tiles
+    assert sum(ns[r] for r in few) < 15000 < sum(ns)
+    off1, j1, f1, a1 = run(few)
+    first = 0
+    for r in few:
+        s, n = start[r], ns[r]
+        o = off[s:s + n + 1]
+        rcs, _ = O.assign_rc(xs[r], boxes[r], table)
+        want, wj = O.build_pairs(xs[r], boxes[r], rcs, 0.3)
+        assert np.array_equal(o - o[0], want) and np.array_equal(j[o[0]:o[-1]] - s, wj)
+        assert np.array_equal(f[s:s + n], f1[first:first + n])
+        assert np.array_equal(a[s:s + n], a1[first:first + n])
+        first += n
