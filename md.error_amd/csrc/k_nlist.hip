@@ -693,13 +693,24 @@ static bool needs_images(const RepInfo &R, float skin) {
 // low mean too, but its lists are a liquid's, more than 60 entries: once such
 // lists have been met, tiles (a gas of 16 entries hardly has one of 40).
 // (b) Boxes so short along z that a tile's window takes in the whole column
-// where its atoms' own do not, which has the tile done atom by atom (liquids in
-// cubes and plates of 2.9 list radii along z): x < 128 and 15 000 atoms, or
-// x < 300 and 20 000.
-//   cube / plate, x = 69 (cutoff 2.5)   16 000 atoms  66.1 / 54.1, 70.6 / 64.0
-//                                      100 000        255 / 96, 238 / 114
-//   x = 260   16 000  103.5 / 89.6, 105.8 / 109.7   100 000  377 / 198, 355 / 259
-//   (plate, x = 470   16 000  125 / 161   100 000  443 / 373   400 000  1149 / 1260)
+// where its atoms' own do not, which has the tile done atom by atom (2.8 to 3.15
+// list radii along z at the default cells; liquids, tiles over windows):
+//                        5 000   11 000   16 000   60 000  100 000  200 000  400 000 atoms
+//   cube of 2.9  x = 69    1.15     1.21     1.23     1.59     2.71     2.82     3.02
+//   (second      x = 250   1.01     1.12     1.13     1.27     1.93     1.86     1.84
+//   images too)  x = 468   1.00     1.09     1.13     1.14     1.75     1.53     1.46
+//                x = 785                     1.08     1.09     1.54     1.31     1.21
+//                x = 1491                    1.00     0.93     1.35     1.13     1.01
+//   plate 6 x 6 x 2.9
+//                x = 69    0.99     1.05     1.10     1.48     2.09     2.09     2.24
+//                x = 113   0.93     0.97     1.01     1.17     1.70     1.66     1.70
+//                x = 172   0.90     0.90     0.94     1.02     1.52     1.51     1.48
+//                x = 250   0.92     0.91     0.97     0.93     1.42     1.29     1.25
+//                x = 347                     0.87     0.81     1.31     1.02     0.97
+//                x = 468   0.97     0.97     0.96     0.79     1.13     0.94     0.83
+// (4 x 4 x 3: 1.14 at x = 172 and 60 000, 1.23 at x = 468 and 100 000; cubes of
+// 3.1 lie near the plates).  With eight atoms a tile spans more of its cell
+// than with four, so more tiles are done atom by atom.
 // (c) Boxes whose atoms see second images (x < 200), or so short along z that a
 // tile's pairs take the exact predicate (x < 500): 40 000 atoms.
 //   cube of 2.1 list radii, x = 69   24 000  50.2 / 46.7   65 000  72.9 / 61.7   400 000  259 / 208
@@ -724,14 +735,24 @@ BuildForm build_form(const RepInfo *reps, int n_rep, float skin, bool dense) {
     const bool column = 2 * (int)ceil(rl / R.h[2]) + 1 < R.nc[2] &&
                         (len + 2.0 * rl) / R.h[2] + 2.0 > R.nc[2];
     const bool flat = 0.3 * R.h[2] > 0.5 * R.L[2] - rl;
+    const double most_x = second ? (atoms < 6000.0       ? 0.0
+                                    : atoms < kTileAtoms ? 1000.0
+                                                         : 1500.0)
+                                 : (atoms < 10000.0      ? 0.0
+                                    : atoms < 20000.0    ? 100.0
+                                    : atoms < 40000.0    ? 128.0
+                                    : atoms < kTileAtoms ? 200.0
+                                    : atoms < 150000.0   ? 500.0
+                                                         : 400.0);
+    const bool own = column && x < most_x;
     if (x < 16.0 && !dense) dilute += R.n_atoms;
-    if (column && (x < 128.0 || (x < 300.0 && atoms >= 20000.0))) whole += R.n_atoms;
-    if ((second && x < 200.0) || (column && x < 300.0) || (flat && x < 500.0)) small += R.n_atoms;
+    if (own) whole += R.n_atoms;
+    if ((second && x < 200.0) || own || (flat && x < 500.0)) small += R.n_atoms;
     images |= second;
   }
   const double most = 0.5 * atoms;
   if (atoms >= 40000.0 && (dilute > most || small > most)) return BuildForm::kSparse;
-  if (atoms >= 15000.0 && whole > most) return BuildForm::kSparse;
+  if (whole > most) return BuildForm::kSparse;
   return images ? BuildForm::kImages : BuildForm::kTiles;
 }
 

@@ -132,6 +132,8 @@ BATCHES = [
     [((7.3, 22.0, 22.0), 2.5, 18)],
     [((16.8, 16.8, 5.75), 2.5, 38)],
     [((11.0, 11.1, 11.05), 3.5, 21)],
+    [((15.45, 15.45, 15.45), 5.0, 6)],
+    [((16.55, 16.6, 16.55), 5.0, 25)],          # above 80 000 atoms
     [((8.1, 8.1, 8.1), 2.5, 40), ((14.0, 14.0, 14.0), 2.5, 3)],
     [((8.1, 8.1, 8.1), 2.5, 20), ((14.0, 14.0, 14.0), 2.5, 6)],
 ]
@@ -168,7 +170,7 @@ def test_batches_of_small_boxes(torch_cuda, batch, lanes):
     R = len(ns)
     off, j, f, a = run(range(R))
     start = np.concatenate([[0], np.cumsum(ns)])
-    few = sorted({0, 1, R - 1})            # a batch of fewer than 15 000 atoms: tiles
+    few = sorted({0, 1, R - 1})            # a small batch: by tiles in all but one of the cases
     assert sum(ns[r] for r in few) < 15000 < sum(ns)
     off1, j1, f1, a1 = run(few)
     first = 0
