@@ -228,23 +228,29 @@ sre_status sre_adjoint(sre_engine *e, const double *dLdE, const double *d_dLdF,
 typedef struct {
   int force_lanes;      /* lanes per atom in the force kernel: 1,2,4,8,16 */
   int build_lanes;      /* 1,2,4,8,16; kept for callers that set it: the list build
-                           takes a few atoms per wavefront at any value */
-  int block;            /* threads per block of the force kernel: 64..1024 */
+                           takes a few atoms per wavefront at any value (another
+                           value still drops the list, as any layout field) */
+  int block;            /* threads per block of the force kernel: 64, 128, 256 */
   float cell_xy;        /* cell edge in x,y as a multiple of (rc_min + skin) */
   float cell_z;         /* cell edge in z as a multiple of (rc_min + skin) */
   int build_mode;       /* 0: column search, 4 or 8 atoms per wavefront on the matrix
                            cores; 1: one wavefront per 64-atom tile of a cell column */
   int xcd_remap;        /* 1: map contiguous atom ranges to each XCD (L2 locality) */
   int force_unroll;     /* list rows per group in the mixed force kernel: 1, 2, 4
-                           (the FP64 form takes one row per group at any value) */
+                           (the FP64 form takes one row per group at any value).
+                           Small systems without statistics -- at most one tile of
+                           64/force_lanes atoms per SIMD, persistent 0 -- run four
+                           wavefronts per tile with two rows per group, whatever
+                           block and force_unroll say; the sums are the same */
   int persistent;       /* mixed force kernel: 0 = one wavefront per tile of 64/lanes
                            atoms (flat launch over all replicas); k = 1..16: a
                            persistent launch of k wavefronts per SIMD, each taking a
                            contiguous chunk of tiles (same sums) */
   int sort_mode;        /* binning at a rebuild (same cell order in every mode):
-                           0 = counting sort by cell up to 30720 cells, radix sort
-                           above; 1 = LSD radix sort of the cell key; 2 = counting
-                           sort at any cell count */
+                           0 = counting sort by cell up to 30720 cells (15360 with
+                           more than 16 atoms per cell), radix sort above; 1 = LSD
+                           radix sort of the cell key; 2 = counting sort at any
+                           cell count */
   int force_mode;       /* mixed form: 0 = neighbor-list kernel; 1 = cell-window
                            kernel without a list (one wavefront per 16-atom tile of
                            a cell column, four lanes per atom, candidates staged in

@@ -11,8 +11,9 @@
 // single-block kernel (or, in small systems, every block of the next drift)
 // turns the reduced sums into the velocity factors of the next step
 // (v <- a2 (a1 v - v_com)), using that scaling all velocities by a multiplies K
-// by a^2 and that removing the COM velocity lowers K by |P|^2 / 2M.  The drift is also the position refresh.  No host
-// synchronisation: the whole step is graph-capturable.
+// by a^2 and that removing the COM velocity lowers K by |P|^2 / 2M.  The drift is
+// also the position refresh.  No host synchronisation: the whole step is
+// graph-capturable.
 #include "sre_internal.h"
 
 namespace sre {

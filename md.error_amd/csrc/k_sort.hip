@@ -9,13 +9,13 @@
 //     k_cell_count), whose atomics only place atoms in a cell's slots before
 //     a rank by caller index fixes their order;
 //   * an atomic-free LSD radix sort of the cell key over digits of at most 8
-//     bits (the allocation-free path and a tuning option), each pass built
-//     from (1) a per-block stable ranking of 1024 keys: lanes holding the
-//     same digit find each other with one ballot per digit bit (their rank is
-//     the number of such lanes below them), per-wave digit counts go through
-//     LDS, and the keys are written in (digit, original position) order;
-//     (2) a digit-major exclusive scan of the per-block digit counts; (3) a
-//     stable scatter to the global positions.
+//     bits (larger cell grids, and a tuning option), each pass built from
+//     (1) a per-block stable ranking of 1024 keys: lanes holding the same
+//     digit find each other with one ballot per digit bit (their rank is the
+//     number of such lanes below them), per-wave digit counts go through LDS,
+//     and the keys are written in (digit, original position) order; (2) a
+//     digit-major exclusive scan of the per-block digit counts; (3) a stable
+//     scatter to the global positions.
 #include "sre_internal.h"
 
 namespace sre {
