@@ -680,8 +680,8 @@ static bool needs_images(const RepInfo &R, float skin) {
   return false;
 }
 
-// Windows per atom where a rebuild is faster with them, for most of the atoms of
-// a large system.  x = list entries per atom at the mean density and the
+// Windows per atom where a rebuild is faster with them for the batch as a whole.
+// x = list entries per atom at the mean density and the
 // replica's largest cutoff; rebuild with tiles / with windows per atom, us.
 // (a) Dilute: x < 16 and 40 000 atoms (uniform and graded cutoffs of 2.5 to 5).
 //   16 000 atoms   x = 3.3  70.5 / 71.6    x = 12.5   71.3 / 76.2   x = 23   48.5 / 56.0
@@ -710,7 +710,11 @@ static bool needs_images(const RepInfo &R, float skin) {
 //                x = 468   0.97     0.97     0.96     0.79     1.13     0.94     0.83
 // (4 x 4 x 3: 1.14 at x = 172 and 60 000, 1.23 at x = 468 and 100 000; cubes of
 // 3.1 lie near the plates).  With eight atoms a tile spans more of its cell
-// than with four, so more tiles are done atom by atom.
+// than with four, so more tiles are done atom by atom.  A batch of 80 000 atoms
+// in which such boxes hold a part only, the rest in cubes of 5:
+//   cube of 2.9, x = 69   100 000 atoms: a quarter 1.11, 45 % 1.37   300 000: 1.14, 1.39
+//   4 x 4 x 3,   x = 250  100 000        a quarter 1.11, 45 % 1.26   300 000: 0.94, 1.08
+// (60 000 atoms: 0.83 to 1.13); so from a quarter of the atoms on, else a half.
 // (c) Boxes whose atoms see second images (x < 200), or so short along z that a
 // tile's pairs take the exact predicate (x < 500): 40 000 atoms.
 //   cube of 2.1 list radii, x = 69   24 000  50.2 / 46.7   65 000  72.9 / 61.7   400 000  259 / 208
@@ -752,7 +756,7 @@ BuildForm build_form(const RepInfo *reps, int n_rep, float skin, bool dense) {
   }
   const double most = 0.5 * atoms;
   if (atoms >= 40000.0 && (dilute > most || small > most)) return BuildForm::kSparse;
-  if (whole > most) return BuildForm::kSparse;
+  if (whole > (atoms < kTileAtoms ? most : 0.25 * atoms)) return BuildForm::kSparse;
   return images ? BuildForm::kImages : BuildForm::kTiles;
 }
 

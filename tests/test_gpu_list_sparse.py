@@ -136,6 +136,7 @@ BATCHES = [
     [((16.55, 16.6, 16.55), 5.0, 25)],          # above 80 000 atoms
     [((8.1, 8.1, 8.1), 2.5, 40), ((14.0, 14.0, 14.0), 2.5, 3)],
     [((8.1, 8.1, 8.1), 2.5, 20), ((14.0, 14.0, 14.0), 2.5, 6)],
+    [((8.1, 8.1, 8.1), 2.5, 91), ((14.0, 14.0, 14.0), 2.5, 32)],   # a third, 80 000
 ]
 
 
