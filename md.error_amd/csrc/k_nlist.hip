@@ -681,8 +681,8 @@ static bool needs_images(const RepInfo &R, float skin) {
 }
 
 // Windows per atom where a rebuild is faster with them for the batch as a whole.
-// x = list entries per atom at the mean density and the
-// replica's largest cutoff; rebuild with tiles / with windows per atom, us.
+// x = list entries per atom at the mean density and the replica's largest cutoff;
+// rebuild with tiles / with windows per atom, us.
 // (a) Dilute: x < 16 and 40 000 atoms (uniform and graded cutoffs of 2.5 to 5).
 //   16 000 atoms   x = 3.3  70.5 / 71.6    x = 12.5   71.3 / 76.2   x = 23   48.5 / 56.0
 //   40 000         x = 3.3  74.0 / 69.8    x = 12.5   85.3 / 82.6   x = 23   76.0 / 75.4

@@ -9,6 +9,7 @@ import pytest
 
 from oracle import oracle as O
 from sre import Engine
+from sre.engine import forces_static
 
 pytestmark = pytest.mark.gpu
 
@@ -184,3 +185,30 @@ def test_batches_of_small_boxes(torch_cuda, batch, lanes):
         assert np.array_equal(f[s:s + n], f1[first:first + n])
         assert np.array_equal(a[s:s + n], a1[first:first + n])
         first += n
+
+
+@pytest.mark.parametrize("n", [6003, 5997])     # both sides of the rule
+def test_allocation_free_call(torch_cuda, n):
+    torch = torch_cuda
+    box = np.array([12.47, 51.6, 12.47], np.float32)
+    c = np.array([11, 50, 11])
+    rng = np.random.default_rng(n)
+    s = np.stack(np.unravel_index(rng.permutation(np.prod(c))[:n], c), 1)
+    xyz = np.zeros((n, 4), np.float32)
+    xyz[:, :3] = np.mod((s + 0.5 + rng.uniform(-0.07, 0.07, (n, 3))) * (box / c), box)
+    table = np.array([4.0], np.float32)
+    x = torch.from_numpy(xyz).cuda()
+    torch.cuda.synchronize()
+    e = engine([n], [box], table.reshape(1, 1, 1), "mixed", 4)
+    e.upload_positions(xyz)
+    e.rebuild()
+    off, j = e.export_pairs()
+    rc, _ = O.assign_rc(xyz, box, table.reshape(1, 1, 1))
+    want, wj = O.build_pairs(xyz, box, rc, 0.3)
+    assert np.array_equal(off, want) and np.array_equal(j, wj)
+    e.compute(stats=True)
+    f, stats = e.forces(), e.stats()[0]
+    e.close()
+    F, st = forces_static(x, box, table, skin=0.3, eps=0.1 * ONE, sigma=ONE)
+    torch.cuda.synchronize()
+    assert np.array_equal(F.cpu().numpy(), f) and np.array_equal(np.asarray(st), stats)
